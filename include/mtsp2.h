@@ -389,11 +389,11 @@ int mt_set_spmv_variant(mt_ctx *ctx, int variant, int layers_per_segment);
  * per single-wave persistent workgroup with the next item prefetched into
  * registers; 4 = four systems of one tile per workgroup sharing the tile's
  * couplings in LDS; 5 = the same with the lean LDS layout (three workgroups
- * per CU); 6 (default) = for the inner solves on bricks, persistent
- * four-system workgroups (three per CU) that load their next item while
- * they sweep the current one (elsewhere as 5).  The same operator; 5 and 6
- * round the black tiles' backward sweep differently from 1 and 4 (6 is
- * bitwise 5).  No counterpart in the reference. */
+ * per CU); 6 (default) = as 5, and in the inner solves on bricks, whose
+ * sweeps are the same register sweeps for every variant, the p-update folded
+ * into the red forward launch (variants 1 to 5 run it apart).  The same
+ * operator; 5 and 6 round the black tiles' backward sweep differently from 1
+ * and 4 (6 is bitwise 5).  No counterpart in the reference. */
 int mt_set_dilu_variant(mt_ctx *ctx, int variant);
 /* Layout of the mixed solver's inner FP32 vectors when they are
  * preconditioned by the red-black DILU with the default SpMV: 2 (default) =

@@ -25,6 +25,7 @@
 #pragma once
 
 #include "mt_dilu.hpp"
+#include "mt_sweep.hpp"
 
 namespace mt {
 
@@ -523,34 +524,46 @@ __global__ __launch_bounds__(kBtThreads, 4) void k_spmv_btp(IterArgs<float, floa
 }
 
 // ------------------------------------------------- red-black DILU on bricks
-// k_dilu_rbl's sweeps (the same LDS layout and level order) on bricked data:
-// a tile's right-hand sides, pivots and the six couplings it uses are
-// contiguous runs.  The red forward sweep leaves w = dinv*y of the red tiles
-// in the output (k_dilu_rbl leaves y): that is what the black tiles take from
-// their red neighbours, and the red backward sweep forms z = w - dinv*(sum of
-// the upper terms), as the black backward sweep does (the same operator as
-// dinv*(y - sum), rounded differently).  A tile reads its neighbours' k- and
-// j-faces from their bricks (a k-face is 512 contiguous bytes, a j-face eight
-// runs of 64) and their i-faces, one value per 64 bytes there, from the
-// packed i-faces (DiluArgs::xf) the other colour wrote: w of the red tiles,
-// z of the black tiles.
+// One tile of one colour for NW systems per workgroup, one wave per system:
+// the tile's right-hand sides, pivots and the six couplings it uses are
+// contiguous runs, swept in registers (mt_sweep.hpp).  The red forward sweep
+// leaves w = dinv*y of the red tiles in the output: that is what the black
+// tiles take from their red neighbours, and the red backward sweep forms
+// z = w - dinv*(sum of the upper terms), as the black backward sweep does.  A
+// tile reads its neighbours' k- and j-faces from their bricks (a k-face is 512
+// contiguous bytes, a j-face eight runs of 64) and their i-faces, one value
+// per 64 bytes there, from the packed i-faces (DiluArgs::xf) the other colour
+// wrote: w of the red tiles, z of the black tiles.  What the neighbouring
+// tiles contribute (black: all six faces before the forward sweep; red: all
+// six before the backward one, the forward one has none) is folded into the
+// right-hand side first, so the sweeps' couplings out of the tile are zero.
+// PU: the red forward sweep of the first application forms the BiCGStab
+// p = r + beta (p - omega v) for its tiles as it loads them.
 // DiluArgs on bricks: coef = the [6][nB] couplings (slots 1..6), cstride =
 // nB, vstride = nB, dinv = [nfreq][nB].
-template <class T, class V, int MODE, int NW, bool ZP = false>
-__global__ __launch_bounds__(64 * NW) void k_dilu_bk(DiluArgs<T, V> a, const TileShape* shp) {
-  constexpr int TX = 8, NP = kRbNP, NU = 8, NLEV = 22, NB = kRbNB;
+// What bounds it: memory at many systems (100x100x60+10, 16 systems: red
+// forward 404 MB in 89 us, black 567 MB in 132 us, red backward 511 MB in 108
+// us, 4.3-4.7 TB/s of a copy's 4.9-5.4; per application 327 us, where sweeps
+// out of an LDS box took 461 with persistent workgroups that loaded their next
+// tile meanwhile), one tile's chain of loads, sweep and stores at few (two
+// systems 56 us against 116; 40x40x30+10 19 against 41).  The sweeps are short
+// enough that four or five workgroups per CU hide the loads without
+// prefetching; the p-update variant needs 98 registers and spills at five.
+template <class T, class V, int MODE, int NW, bool ZP = false, bool PU = false>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? (PU ? 4 : 5) : 1) void k_dilu_bc(DiluArgs<T, V> a) {
+  constexpr int TX = 8, NP = kRbNP, NU = 8;
+  static_assert(!PU || MODE == RB_RED_FWD, "the p-update is folded into the red forward sweep");
   constexpr bool FWDP = MODE != RB_RED_BWD;   // has a forward sweep
   constexpr bool BWDP = MODE != RB_RED_FWD;   // has a backward sweep
   constexpr bool HALO = MODE != RB_RED_FWD;   // reads face neighbours
-  struct Cpl { V c[3]; };
-  __shared__ C2<T> Wall[NW][NB];                 // per system: the box
-  // per-point data by level slot (TileShape::rslot)
-  __shared__ C2<T> DVall[NW][NP];                // per system: pivots (red forward: then y)
-  __shared__ Cpl CL[FWDP ? NP : 1];              // raw lower couplings (slots 1, 3, 5)
-  __shared__ Cpl CH[BWDP ? NP : 1];              // raw upper couplings (slots 2, 4, 6)
-  __shared__ int s_sys[NW], s_ok[NW], s_fidx[NW];
-  __shared__ C2<T> s_al[NW];
-  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+  constexpr int CPT = NP / (64 * NW);         // tile points per thread for the couplings
+  __shared__ C2<T> Pall[NW][NP];              // per system: the tile, point order
+  __shared__ C2<T> Xall[NW][64];              // per system: cross-row words of the sweeps
+  // couplings inside the tile (0 across its faces), and across its faces
+  __shared__ V CL[FWDP ? 3 : 1][FWDP ? NP : 1], CH[BWDP ? 3 : 1][BWDP ? NP : 1];
+  __shared__ V FC[HALO ? 6 : 1][64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ngrp = (a.nact + NW - 1) / NW;
   const int nwork = a.ntiles * ngrp;
   const int xcd = blockIdx.x & 7, lb = blockIdx.x >> 3;
@@ -558,23 +571,12 @@ __global__ __launch_bounds__(64 * NW) void k_dilu_bk(DiluArgs<T, V> a, const Til
   const int w = xcd * chunk + lb;
   if (lb >= chunk || w >= nwork) return;   // uniform over the workgroup
   const int tix = w / ngrp, grp = w - tix * ngrp;
-  if (tid < NW) {
-    const int si = grp * NW + tid;
-    int sy = 0, ok = 0, fi = 0;
-    C2<T> al = {T(0), T(0)};
-    if (si < a.nact) {
-      sy = a.act[si];
-      const SysScal& sc = a.sc[sy];
-      ok = sc.status == a.status_req;
-      fi = sc.fidx;
-      al = ccast<T>(sc.alpha);
-    }
-    s_sys[tid] = sy;
-    s_ok[tid] = ok;
-    s_fidx[tid] = fi;
-    s_al[tid] = al;
-  }
+  const int si = grp * NW + wv;
+  const int sys = a.act[si < a.nact ? si : 0];
   const int4 tl = a.tiles[tix];
+  const SysScal& sc = a.sc[sys];
+  const bool mine = si < a.nact && sc.status == a.status_req;   // uniform over the wave
+  const int fidx = sc.fidx;
   const LatticeInfo L = a.lat[tl.x];
   const int gi0 = tl.y * TX, gj0 = tl.z * TX, gk0 = tl.w * TX;
   const int ex = min(TX, L.A - gi0), ey = min(TX, L.B - gj0), ez = min(TX, L.C - gk0);
@@ -582,368 +584,43 @@ __global__ __launch_bounds__(64 * NW) void k_dilu_bk(DiluArgs<T, V> a, const Til
   const int tb = tself * kBkPts;   // the tile's first brick index
   const V* __restrict__ cfs = a.coef;
   const int64_t cst = a.cstride;
-  const int st[3] = {1, kRbBX, kRbPK};
-  // ---- the tile's couplings, once for the NW systems
-  for (int p = tid; p < NP; p += 64 * NW) {
-    const int sl = shp->rslot[p];
-    Cpl c, h;
-#pragma unroll
-    for (int s = 0; s < 3; ++s) {
-      c.c[s] = FWDP ? cfs[(int64_t)(2 * s) * cst + tb + p] : V(0);
-      h.c[s] = BWDP ? cfs[(int64_t)(2 * s + 1) * cst + tb + p] : V(0);
-    }
-    if (FWDP) CL[sl] = c;
-    if (BWDP) CH[sl] = h;
-  }
-  __syncthreads();   // s_ tables
-  // this lane's point on every hyperplane of the tile (at most 48 per plane),
-  // formed before the sweeps: box index | level slot << 10, or ~0u (no point,
-  // or past a partial tile's extent)
-  unsigned int pk[NLEV];
-#pragma unroll
-  for (int h = 0; h < NLEV; ++h) pk[h] = shp->lpts[h][lane];
-#pragma unroll
-  for (int h = 0; h < NLEV; ++h) {
-    const unsigned int v = pk[h];
-    const int li = v & 7, lj = (v >> 3) & 7, lk = (v >> 6) & 7;
-    const bool ok = v != 0xffffffffu && li < ex && lj < ey && lk < ez;
-    pk[h] = ok ? (unsigned(rb_box(li, lj, lk)) | ((v >> 9) << 10)) : 0xffffffffu;
-    asm volatile("" : "+v"(pk[h]));   // formed here, not per sweep step
-  }
-  const bool mine = __builtin_amdgcn_readfirstlane(s_ok[wv]) != 0;   // 0 past nact
-  const int sys = __builtin_amdgcn_readfirstlane(s_sys[wv]);
-  const int fidx = __builtin_amdgcn_readfirstlane(s_fidx[wv]);
-  C2<T>* __restrict__ W = Wall[wv];
-  C2<T>* __restrict__ DV = DVall[wv];
   const int64_t o = (int64_t)sys * a.vstride;
-  // the other colour's results (red backward with zout: the black tiles' z,
-  // pair-interleaved)
-  // (ZP: the launch has a.zout)
+  const int fa = lane & 7, fb = lane >> 3;
   constexpr bool zp = ZP && MODE != RB_RED_FWD;
   constexpr int zs = zp ? 2 : 1;
-  const C2<T>* __restrict__ pout =
-      (MODE == RB_RED_BWD && zp) ? a.zout + (int64_t)(sys >> 1) * a.zpair + (sys & 1) : a.out + o;
-  const C2<T>* __restrict__ xfi =
-      a.xf + (MODE == RB_BLACK_FB ? 0 : a.xfhalf) + (int64_t)sys * a.xfsys;   // faces read
-  C2<T>* __restrict__ xfw =
-      a.xf + (MODE == RB_RED_FWD ? 0 : a.xfhalf) + (int64_t)sys * a.xfsys;    // faces written
-  // face values kept for the fold (black: the high faces; red backward: the
-  // low faces and the lower couplings of the tile points next to them)
-  C2<T> fold_v[3];
-  T fold_c[3];
+  C2<T>* __restrict__ P = Pall[wv];
+  // ---- every load of the item
+  V cl[CPT][3], ch[CPT][3];
 #pragma unroll
-  for (int s = 0; s < 3; ++s) {
-    fold_v[s] = {T(0), T(0)};
-    fold_c[s] = T(0);
+  for (int c = 0; c < CPT; ++c) {
+    const int p = tid + 64 * NW * c;
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      cl[c][s] = FWDP ? cfs[(int64_t)(2 * s) * cst + tb + p] : V(0);
+      ch[c][s] = BWDP ? cfs[(int64_t)(2 * s + 1) * cst + tb + p] : V(0);
+    }
   }
+  // the tile point next to face f (dir = f/2, low or high) for this lane
+  auto face_point = [&](int f) {
+    const int dir = f >> 1, t = (f & 1) ? TX - 1 : 0;
+    if (dir == 0) return t + TX * (fa + TX * fb);
+    if (dir == 1) return fa + TX * (t + TX * fb);
+    return fa + TX * (fb + TX * t);
+  };
+  constexpr int FPW = HALO ? (6 + NW - 1) / NW : 1;   // faces per wave
+  V fcv[FPW];
+  if (HALO) {
+#pragma unroll
+    for (int q = 0; q < FPW; ++q) {
+      const int f = wv + NW * q;
+      fcv[q] = f < 6 ? cfs[(int64_t)f * cst + tb + face_point(f)] : V(0);
+    }
+  }
+  C2<T> rv[NU], v2[NU], r3[PU ? NU : 1], dd[NU], fv[6];
   if (mine) {
-    for (int q = lane; q < NB; q += 64) W[q] = {T(0), T(0)};
     const C2<T>* __restrict__ pin = (FWDP ? a.in : a.out) + o + tb;
     const C2<T>* __restrict__ pin2 = a.in2 ? a.in2 + o + tb : nullptr;
     const C2<T>* __restrict__ dinv = a.dinv + (int64_t)fidx * cst + tb;
-    const C2<T> al = s_al[wv];
-    C2<T> rv[NU], v2[NU], dd[NU];
-#pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      const int p = lane + 64 * u;
-      // points past a partial tile's extent hold zeros
-      rv[u] = pin[p];
-      v2[u] = (FWDP && pin2) ? pin2[p] : C2<T>{T(0), T(0)};
-      dd[u] = dinv[p];
-    }
-    C2<T> fv[6];
-    if (HALO) {
-      const int fa = lane & 7, fb = lane >> 3;
-#pragma unroll
-      for (int f = 0; f < 6; ++f) {
-        const int dir = f >> 1;
-        const bool hi = f & 1;
-        int ti, tj, tk;   // tile point next to the face
-        if (dir == 0) { ti = hi ? 7 : 0; tj = fa; tk = fb; }
-        else if (dir == 1) { ti = fa; tj = hi ? 7 : 0; tk = fb; }
-        else { ti = fa; tj = fb; tk = hi ? 7 : 0; }
-        const int ni = gi0 + ti + (dir == 0 ? (hi ? 1 : -1) : 0);
-        const int nj = gj0 + tj + (dir == 1 ? (hi ? 1 : -1) : 0);
-        const int nk = gk0 + tk + (dir == 2 ? (hi ? 1 : -1) : 0);
-        fv[f] = {T(0), T(0)};
-        const bool pin_ok = ti < ex && tj < ey && tk < ez;
-        const bool ok = pin_ok && ni >= 0 && nj >= 0 && nk >= 0 && ni < L.A && nj < L.B && nk < L.C;
-        if (ok) {
-          // the neighbour tile's facing face: the i-faces packed (entry
-          // tj + 8*tk = lane), the j- and k-faces from the neighbour's brick
-          const int d = hi ? 1 : -1;
-          const int tn = L.tbase + (tl.y + (dir == 0 ? d : 0)) +
-                         L.ntx * ((tl.z + (dir == 1 ? d : 0)) + L.nty * (tl.w + (dir == 2 ? d : 0)));
-          if (dir == 0) {
-            fv[f] = xfi[(int64_t)tn * kRbFaces + (hi ? 0 : 1) * 64 + lane];
-          } else {
-            const int fl = hi ? 0 : TX - 1;   // the neighbour's facing layer
-            const int pn = dir == 1 ? ti + TX * (fl + TX * tk) : ti + TX * (tj + TX * fl);
-            fv[f] = pout[(MODE == RB_RED_BWD ? zs : 1) * ((int64_t)tn * kBkPts + pn)];
-          }
-        }
-        if (MODE == RB_RED_BWD && !hi && pin_ok)
-          fold_c[dir] = T(cfs[(int64_t)(2 * dir) * cst + tb + ti + TX * (tj + TX * tk)]);
-      }
-    }
-    // ---- stage into LDS: the right-hand side in the box, the pivots
-#pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      const int p = lane + 64 * u;
-      const int li = p & 7, lj = (p >> 3) & 7, lk = p >> 6;
-      C2<T> r = rv[u];
-      if (FWDP && pin2) {
-        r = csub(r, cmul(al, v2[u]));
-        if (a.sout) a.sout[o + tb + p] = r;
-      }
-      W[rb_box(li, lj, lk)] = r;
-      DV[shp->rslot[p]] = dd[u];
-    }
-    if (HALO) {
-      const int fa = lane & 7, fb = lane >> 3;
-#pragma unroll
-      for (int f = 0; f < 6; ++f) {
-        const int dir = f >> 1;
-        const bool hi = f & 1;
-        int ti, tj, tk;
-        if (dir == 0) { ti = hi ? 7 : 0; tj = fa; tk = fb; }
-        else if (dir == 1) { ti = fa; tj = hi ? 7 : 0; tk = fb; }
-        else { ti = fa; tj = fb; tk = hi ? 7 : 0; }
-        const C2<T> v = fv[f];
-        const bool inbox = (MODE == RB_BLACK_FB) ? !hi : hi;
-        if (!inbox) {
-          fold_v[dir] = v;
-          continue;
-        }
-        if (!(ti < ex && tj < ey && tk < ez)) continue;
-        const int qp = rb_box(ti, tj, tk);
-        int qs = hi ? qp + st[dir] : qp - st[dir];
-        if (qs >= NB) qs -= NB;
-        W[qs] = v;
-      }
-    }
-  }
-  __syncthreads();   // the shared couplings; the rest is per wave
-  if (!mine) return;
-  // fold the face terms the sweeps do not read, one direction after another:
-  // black forward, the high faces (red neighbours above, upper couplings);
-  // red backward, the low faces (black neighbours below, lower couplings)
-  if (HALO) {
-    const int fa = lane & 7, fb = lane >> 3;
-#pragma unroll
-    for (int s = 0; s < 3; ++s) {
-      const int t0 = (MODE == RB_BLACK_FB) ? TX - 1 : 0;
-      int ti, tj, tk;
-      if (s == 0) { ti = t0; tj = fa; tk = fb; }
-      else if (s == 1) { ti = fa; tj = t0; tk = fb; }
-      else { ti = fa; tj = fb; tk = t0; }
-      if (ti < ex && tj < ey && tk < ez) {
-        const int q = rb_box(ti, tj, tk);
-        const int sl = shp->rslot[ti + TX * (tj + TX * tk)];
-        const T c = (MODE == RB_BLACK_FB) ? T(CH[sl].c[s]) : fold_c[s];
-        const C2<T> v = fold_v[s];
-        C2<T> r = W[q];
-        if (MODE == RB_BLACK_FB) {
-          r.x -= c * v.x;
-          r.y -= c * v.y;
-        } else {
-          // the box holds w = dinv*y: subtract dinv*(c v)
-          const C2<T> d = cmul(DV[sl], C2<T>{c * v.x, c * v.y});
-          r.x -= d.x;
-          r.y -= d.y;
-        }
-        W[q] = r;
-      }
-      wave_sync();
-    }
-  }
-  // The sweeps take no masks: a red forward step's low neighbours outside the
-  // tile are zero cells of the box (red forward stages no faces); a black
-  // point uses every lower coupling; before the black backward sweep the
-  // low-face cells are cleared, so that every upper neighbour outside the
-  // tile (an i-high cell is the next row's i-low cell, a j-high cell the next
-  // plane's j-low cells, a k-high index wraps to the k-low plane) reads zero;
-  // red backward uses every upper coupling with the high faces in the box.
-  // A neighbour past a partial tile's extent is a pad point: zero.
-  if (FWDP) {
-#pragma unroll
-    for (int h = 0; h < NLEV; ++h) {
-      const unsigned int pt = pk[h];
-      if (pt != 0xffffffffu) {
-        const int q = pt & 0x3ff, p = pt >> 10;
-        const C2<T> dvp = DV[p];
-        const Cpl c4 = CL[p];
-        C2<T> y = W[q];
-        C2<T> v[3];
-#pragma unroll
-        for (int s = 0; s < 3; ++s) v[s] = W[q - st[s]];
-#pragma unroll
-        for (int s = 0; s < 3; ++s) {
-          const T c = T(c4.c[s]);
-          y.x -= c * v[s].x;
-          y.y -= c * v[s].y;
-        }
-        W[q] = cmul(dvp, y);
-      }
-      wave_sync();
-    }
-  }
-  if (MODE == RB_BLACK_FB) {
-    const int fa = lane & 7, fb = lane >> 3;
-    W[rb_box(0, fa, fb) - 1] = {T(0), T(0)};
-    W[rb_box(fa, 0, fb) - kRbBX] = {T(0), T(0)};
-    W[rb_box(fa, fb, 0) - kRbPK] = {T(0), T(0)};
-    wave_sync();
-  }
-  if (BWDP) {
-#pragma unroll
-    for (int h = NLEV - 1; h >= 0; --h) {
-      const unsigned int pt = pk[h];
-      if (pt != 0xffffffffu) {
-        const int q = pt & 0x3ff, p = pt >> 10;
-        const C2<T> dvp = DV[p];
-        const Cpl h4 = CH[p];
-        const C2<T> b = W[q];
-        C2<T> z[3];
-#pragma unroll
-        for (int s = 0; s < 3; ++s) {
-          // q + st < 2 NB: the index past the box wraps to its start
-          const unsigned int qn = unsigned(q + st[s]);
-          z[s] = W[s == 0 ? qn : min(qn, qn - unsigned(NB))];
-        }
-        // y = -(sum of the upper terms); the box holds w = dv*y_forward
-        C2<T> y = {T(0), T(0)};
-#pragma unroll
-        for (int s = 0; s < 3; ++s) {
-          const T c = T(h4.c[s]);
-          y.x -= c * z[s].x;
-          y.y -= c * z[s].y;
-        }
-        const C2<T> d = cmul(dvp, y);
-        W[q] = {b.x + d.x, b.y + d.y};
-      }
-      wave_sync();
-    }
-  }
-  // ---- write the tile back (red forward: y; otherwise z) and the packed
-  // faces the other colour reads next (red forward: dinv*y; black: z)
-  C2<T>* __restrict__ dst =
-      zp ? a.zout + (int64_t)(sys >> 1) * a.zpair + (sys & 1) + 2 * (int64_t)tb : a.out + o + tb;
-  C2<T>* __restrict__ xfo = xfw + (int64_t)tself * kRbFaces;
-  for (int p = lane; p < NP; p += 64) {
-    const int li = p & 7, lj = (p >> 3) & 7, lk = p >> 6;
-    if (!(li < ex && lj < ey && lk < ez)) continue;
-    const int q = rb_box(li, lj, lk);
-    const C2<T> zv = W[q];
-    dst[zs * p] = zv;
-    if (MODE != RB_RED_BWD && (li == 0 || li == TX - 1)) xfo[(li == 0 ? 0 : 64) + lj + 8 * lk] = zv;
-  }
-}
-
-// The same three launches with persistent workgroups: a workgroup walks its
-// XCD's items (tile, group of NW systems) with a stride, and while the waves
-// sweep one item out of LDS, the loads of the next item (right-hand sides,
-// pivots, couplings, faces; the system records and the tile before them) are
-// in flight into registers.  The sweeps leave the loads little to overlap
-// with otherwise: a workgroup's tile data arrive in one burst and the memory
-// pipe idles while its waves sweep.  The arithmetic is k_dilu_bk's.
-template <class T, class V, int MODE, int NW, bool ZP = false, bool PU = false>
-__global__ __launch_bounds__(64 * NW) void k_dilu_bkp(DiluArgs<T, V> a, const TileShape* shp) {
-  constexpr int TX = 8, NP = kRbNP, NU = 8, NLEV = 22, NB = kRbNB;
-  static_assert(!PU || MODE == RB_RED_FWD, "the p-update is folded into the red forward sweep");
-  constexpr bool FWDP = MODE != RB_RED_BWD;   // has a forward sweep
-  constexpr bool BWDP = MODE != RB_RED_FWD;   // has a backward sweep
-  constexpr bool HALO = MODE != RB_RED_FWD;   // reads face neighbours
-  constexpr int CPT = NP / (64 * NW);         // tile points per thread for the couplings
-  static_assert(CPT * 64 * NW == NP, "couplings: whole points per thread");
-  struct Cpl { V c[3]; };
-  __shared__ C2<T> Wall[NW][NB];
-  __shared__ C2<T> DVall[NW][NP];
-  __shared__ Cpl CL[FWDP ? NP : 1];
-  __shared__ Cpl CH[BWDP ? NP : 1];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ngrp = (a.nact + NW - 1) / NW;
-  const int nwork = a.ntiles * ngrp;
-  const int xcd = blockIdx.x & 7, nb8 = gridDim.x >> 3;
-  const int chunk = (nwork + 7) / 8;
-  const int wend = min(nwork, (xcd + 1) * chunk);
-  int w = xcd * chunk + (blockIdx.x >> 3);
-  if (w >= wend) return;   // uniform over the workgroup
-  C2<T>* __restrict__ W = Wall[wv];
-  C2<T>* __restrict__ DV = DVall[wv];
-  const V* __restrict__ cfs = a.coef;
-  const int64_t cst = a.cstride;
-  const int st[3] = {1, kRbBX, kRbPK};
-  const int fa = lane & 7, fb = lane >> 3;
-  // constant over the items: the lane's point of every hyperplane (box index
-  // | level slot << 10 | li << 19 | lj << 22 | lk << 25, or ~0u), the level
-  // slots of its staging points and of its coupling points
-  unsigned int pk[NLEV];
-#pragma unroll
-  for (int h = 0; h < NLEV; ++h) {
-    const unsigned int v = shp->lpts[h][lane];
-    const unsigned int li = v & 7, lj = (v >> 3) & 7, lk = (v >> 6) & 7;
-    pk[h] = v == 0xffffffffu ? v
-                             : (unsigned(rb_box(li, lj, lk)) | ((v >> 9) << 10) | (li << 19) | (lj << 22) |
-                                (lk << 25));
-  }
-  int sl[NU], csl[CPT];
-#pragma unroll
-  for (int u = 0; u < NU; ++u) sl[u] = shp->rslot[lane + 64 * u];
-#pragma unroll
-  for (int c = 0; c < CPT; ++c) csl[c] = shp->rslot[tid + 64 * NW * c];
-  // ---- the prefetched item
-  struct Geo {
-    int ok, sys, fidx, tself, ex, ey, ez;
-    C2<T> al;
-    int rs;           // PU: restart due
-    C2<T> beta, om;   // PU: beta, omega
-  };
-  Geo nx;
-  C2<T> rv[NU], v2[NU], dd[NU], fv[6];
-  C2<T> r3[PU ? NU : 1];   // PU: r
-  V cp[CPT][6];
-  T fc[3];
-  auto load = [&](int wi) {
-    const int tix = wi / ngrp, grp = wi - tix * ngrp;
-    const int si = grp * NW + wv;
-    nx.ok = 0; nx.sys = 0; nx.fidx = 0;
-    nx.al = {T(0), T(0)};
-    if (si < a.nact) {
-      nx.sys = a.act[si];
-      const SysScal& sc = a.sc[nx.sys];
-      nx.ok = sc.status == a.status_req;
-      nx.fidx = sc.fidx;
-      nx.al = ccast<T>(sc.alpha);
-      if constexpr (PU) {
-        nx.rs = sc.restart_due;
-        nx.beta = ccast<T>(sc.beta);
-        nx.om = ccast<T>(sc.omg);
-      }
-    }
-    const int4 tl = a.tiles[tix];
-    const LatticeInfo L = a.lat[tl.x];
-    const int gi0 = tl.y * TX, gj0 = tl.z * TX, gk0 = tl.w * TX;
-    nx.ex = min(TX, L.A - gi0);
-    nx.ey = min(TX, L.B - gj0);
-    nx.ez = min(TX, L.C - gk0);
-    nx.tself = L.tbase + tl.y + L.ntx * (tl.z + L.nty * tl.w);
-    const int tb = nx.tself * kBkPts;
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      const int p = tid + 64 * NW * c;
-#pragma unroll
-      for (int s = 0; s < 3; ++s) {
-        cp[c][s] = FWDP ? cfs[(int64_t)(2 * s) * cst + tb + p] : V(0);
-        cp[c][3 + s] = BWDP ? cfs[(int64_t)(2 * s + 1) * cst + tb + p] : V(0);
-      }
-    }
-    if (!nx.ok) return;
-    const int64_t o = (int64_t)nx.sys * a.vstride;
-    const C2<T>* __restrict__ pin = (FWDP ? a.in : a.out) + o + tb;
-    const C2<T>* __restrict__ pin2 = a.in2 ? a.in2 + o + tb : nullptr;
-    const C2<T>* __restrict__ dinv = a.dinv + (int64_t)nx.fidx * cst + tb;
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       const int p = lane + 64 * u;
@@ -957,239 +634,166 @@ __global__ __launch_bounds__(64 * NW) void k_dilu_bkp(DiluArgs<T, V> a, const Ti
       dd[u] = dinv[p];
     }
     if (HALO) {
-      // the other colour's results (red backward with zout: the black
-      // tiles' z, pair-interleaved)
+      // the other colour's results (red backward with zout: the black tiles'
+      // z, pair-interleaved)
       constexpr bool zr = ZP && MODE == RB_RED_BWD;   // (ZP: the launch has a.zout)
       const C2<T>* __restrict__ pout =
-          zr ? a.zout + (int64_t)(nx.sys >> 1) * a.zpair + (nx.sys & 1) : a.out + o;
-      constexpr int zs = zr ? 2 : 1;
+          zr ? a.zout + (int64_t)(sys >> 1) * a.zpair + (sys & 1) : a.out + o;
       const C2<T>* __restrict__ xfi =
-          a.xf + (MODE == RB_BLACK_FB ? 0 : a.xfhalf) + (int64_t)nx.sys * a.xfsys;
+          a.xf + (MODE == RB_BLACK_FB ? 0 : a.xfhalf) + (int64_t)sys * a.xfsys;
 #pragma unroll
       for (int f = 0; f < 6; ++f) {
-        const int dir = f >> 1;
-        const bool hi = f & 1;
-        int ti, tj, tk;   // tile point next to the face
-        if (dir == 0) { ti = hi ? 7 : 0; tj = fa; tk = fb; }
-        else if (dir == 1) { ti = fa; tj = hi ? 7 : 0; tk = fb; }
-        else { ti = fa; tj = fb; tk = hi ? 7 : 0; }
-        const int ni = gi0 + ti + (dir == 0 ? (hi ? 1 : -1) : 0);
-        const int nj = gj0 + tj + (dir == 1 ? (hi ? 1 : -1) : 0);
-        const int nk = gk0 + tk + (dir == 2 ? (hi ? 1 : -1) : 0);
+        const int dir = f >> 1, d = (f & 1) ? 1 : -1;
+        const int ni = tl.y + (dir == 0 ? d : 0), nj = tl.z + (dir == 1 ? d : 0),
+                  nk = tl.w + (dir == 2 ? d : 0);
         fv[f] = {T(0), T(0)};
-        const bool pin_ok = ti < nx.ex && tj < nx.ey && tk < nx.ez;
-        const bool ok = pin_ok && ni >= 0 && nj >= 0 && nk >= 0 && ni < L.A && nj < L.B && nk < L.C;
-        if (ok) {
-          const int d = hi ? 1 : -1;
-          const int tn = L.tbase + (tl.y + (dir == 0 ? d : 0)) +
-                         L.ntx * ((tl.z + (dir == 1 ? d : 0)) + L.nty * (tl.w + (dir == 2 ? d : 0)));
+        // (uniform) the neighbouring tile exists
+        if (ni >= 0 && nj >= 0 && nk >= 0 && ni * TX < L.A && nj * TX < L.B && nk * TX < L.C) {
+          const int tn = L.tbase + ni + L.ntx * (nj + L.nty * nk);
+          // its facing layer: i-faces packed (entry lj + 8*lk = lane), j- and
+          // k-faces from its brick
+          if (!(fa < (dir == 0 ? ey : ex) && fb < (dir == 2 ? ey : ez))) continue;
           if (dir == 0) {
-            fv[f] = xfi[(int64_t)tn * kRbFaces + (hi ? 0 : 1) * 64 + lane];
+            fv[f] = xfi[(int64_t)tn * kRbFaces + ((f & 1) ? 0 : 64) + lane];
           } else {
-            const int fl = hi ? 0 : TX - 1;   // the neighbour's facing layer
-            const int pn = dir == 1 ? ti + TX * (fl + TX * tk) : ti + TX * (tj + TX * fl);
-            fv[f] = pout[zs * ((int64_t)tn * kBkPts + pn)];
+            const int fl = (f & 1) ? 0 : TX - 1;
+            const int pn = dir == 1 ? fa + TX * (fl + TX * fb) : fa + TX * (fb + TX * fl);
+            fv[f] = pout[(zr ? 2 : 1) * ((int64_t)tn * kBkPts + pn)];
           }
-        }
-        if (MODE == RB_RED_BWD && !hi) {
-          fc[dir] = T(0);
-          if (pin_ok) fc[dir] = T(cfs[(int64_t)(2 * dir) * cst + tb + ti + TX * (tj + TX * tk)]);
         }
       }
     }
-  };
-  load(w);
-  while (true) {
-    // the point table is loop-invariant: kept opaque, so that what the sweeps
-    // derive from it (addresses of 22 levels) is not hoisted out of the loop
-    // into registers
+  }
+  // ---- the couplings into LDS, those across the tile's faces apart
 #pragma unroll
-    for (int h = 0; h < NLEV; ++h) asm volatile("" : "+v"(pk[h]));
-    const Geo cu = nx;
-    const int ex = cu.ex, ey = cu.ey, ez = cu.ez;
-    const bool mine = __builtin_amdgcn_readfirstlane(cu.ok) != 0;
-    __syncthreads();   // the previous item's sweeps and write-back are done
-    // ---- stage: the shared couplings, per wave the box and the pivots
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      if (FWDP) CL[csl[c]] = Cpl{{cp[c][0], cp[c][1], cp[c][2]}};
-      if (BWDP) CH[csl[c]] = Cpl{{cp[c][3], cp[c][4], cp[c][5]}};
-    }
-    C2<T> fold_v[3];
-    T fold_c[3];
+  for (int c = 0; c < CPT; ++c) {
+    const int p = tid + 64 * NW * c;
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
-      fold_v[s] = {T(0), T(0)};
-      fold_c[s] = MODE == RB_RED_BWD ? fc[s] : T(0);
+      const int q = s == 0 ? (p & 7) : (s == 1 ? ((p >> 3) & 7) : (p >> 6));
+      if (FWDP) CL[s][p] = q == 0 ? V(0) : cl[c][s];
+      if (BWDP) CH[s][p] = q == TX - 1 ? V(0) : ch[c][s];
     }
-    if (mine) {
-      for (int q = lane; q < NB; q += 64) W[q] = {T(0), T(0)};
-      wave_sync();
-      C2<T>* __restrict__ so =
-          a.sout ? a.sout + (int64_t)cu.sys * a.vstride + (int64_t)cu.tself * kBkPts : nullptr;
+  }
+  if (HALO) {
 #pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        C2<T> r = rv[u];
-        if constexpr (PU) {
-          // k_pupdate's p, stored for the red tiles
-          const int64_t pe = (int64_t)cu.sys * a.vstride + (int64_t)cu.tself * kBkPts + lane + 64 * u;
-          if (cu.rs) {
-            a.pu_rt[pe] = r3[u];
-            r = r3[u];
-          } else {
-            r = cadd(r3[u], cmul(cu.beta, csub(r, cmul(cu.om, v2[u]))));
-          }
-          a.pu_p[pe] = r;
-        } else if (FWDP && a.in2) {
-          r = csub(r, cmul(cu.al, v2[u]));
-          if (so) so[lane + 64 * u] = r;
-        }
-        W[rb_box(fa, fb & 7, u)] = r;
-        DV[sl[u]] = dd[u];
-      }
-      if (HALO) {
-#pragma unroll
-        for (int f = 0; f < 6; ++f) {
-          const int dir = f >> 1;
-          const bool hi = f & 1;
-          int ti, tj, tk;
-          if (dir == 0) { ti = hi ? 7 : 0; tj = fa; tk = fb; }
-          else if (dir == 1) { ti = fa; tj = hi ? 7 : 0; tk = fb; }
-          else { ti = fa; tj = fb; tk = hi ? 7 : 0; }
-          const bool inbox = (MODE == RB_BLACK_FB) ? !hi : hi;
-          if (!inbox) {
-            fold_v[dir] = fv[f];
-            continue;
-          }
-          if (!(ti < ex && tj < ey && tk < ez)) continue;
-          const int qp = rb_box(ti, tj, tk);
-          int qs = hi ? qp + st[dir] : qp - st[dir];
-          if (qs >= NB) qs -= NB;
-          W[qs] = fv[f];
-        }
-      }
+    for (int q = 0; q < FPW; ++q) {
+      const int f = wv + NW * q;
+      if (f < 6) FC[f][lane] = fcv[q];
     }
-    // ---- the next item's loads, in flight during this item's sweeps
-    const int wn = w + nb8;
-    const bool more = wn < wend;
-    if (more) load(wn);
-    __syncthreads();   // the shared couplings
-    if (mine) {
-      const int64_t o = (int64_t)cu.sys * a.vstride;
-      // fold the face terms the sweeps do not read (k_dilu_bk)
-      if (HALO) {
+  }
+  __syncthreads();   // the shared couplings; the rest is per wave
+  if (!mine) return;
+  const int skew = sw_skew(lane);
+  const C2<T> zero = {T(0), T(0)};
+  // ---- pivots, through the tile buffer into skewed registers
+  C2<T> D[NU], R[NU];
 #pragma unroll
-        for (int s = 0; s < 3; ++s) {
-          const int t0 = (MODE == RB_BLACK_FB) ? TX - 1 : 0;
-          int ti, tj, tk;
-          if (s == 0) { ti = t0; tj = fa; tk = fb; }
-          else if (s == 1) { ti = fa; tj = t0; tk = fb; }
-          else { ti = fa; tj = fb; tk = t0; }
-          if (ti < ex && tj < ey && tk < ez) {
-            const int q = rb_box(ti, tj, tk);
-            const int sq = shp->rslot[ti + TX * (tj + TX * tk)];
-            const T c = (MODE == RB_BLACK_FB) ? T(CH[sq].c[s]) : fold_c[s];
-            const C2<T> v = fold_v[s];
-            C2<T> r = W[q];
-            if (MODE == RB_BLACK_FB) {
-              r.x -= c * v.x;
-              r.y -= c * v.y;
-            } else {
-              const C2<T> d = cmul(DV[sq], C2<T>{c * v.x, c * v.y});
-              r.x -= d.x;
-              r.y -= d.y;
-            }
-            W[q] = r;
-          }
-          wave_sync();
-        }
-      }
-      const bool full = ex == TX && ey == TX && ez == TX;
-      auto live = [&](unsigned int pt) {
-        return pt != 0xffffffffu &&
-               (full || (int((pt >> 19) & 7) < ex && int((pt >> 22) & 7) < ey && int((pt >> 25) & 7) < ez));
-      };
-      if (FWDP) {
+  for (int u = 0; u < NU; ++u) P[lane + 64 * u] = dd[u];
+  Xall[wv][lane] = zero;
+  sw_order();
 #pragma unroll
-        for (int h = 0; h < NLEV; ++h) {
-          const unsigned int pt = pk[h];
-          if (live(pt)) {
-            const int q = pt & 0x3ff, p = (pt >> 10) & 0x1ff;
-            const C2<T> dvp = DV[p];
-            const Cpl c4 = CL[p];
-            C2<T> y = W[q];
-            C2<T> v[3];
+  for (int u = 0; u < NU; ++u) D[u] = P[sw_point(lane, skew, u)];
+  if (HALO) {
 #pragma unroll
-            for (int s = 0; s < 3; ++s) v[s] = W[q - st[s]];
-#pragma unroll
-            for (int s = 0; s < 3; ++s) {
-              const T c = T(c4.c[s]);
-              y.x -= c * v[s].x;
-              y.y -= c * v[s].y;
-            }
-            W[q] = cmul(dvp, y);
-          }
-          wave_sync();
-        }
-      }
-      if (MODE == RB_BLACK_FB) {
-        W[rb_box(0, fa, fb) - 1] = {T(0), T(0)};
-        W[rb_box(fa, 0, fb) - kRbBX] = {T(0), T(0)};
-        W[rb_box(fa, fb, 0) - kRbPK] = {T(0), T(0)};
-        wave_sync();
-        // nothing the forward sweep derived from the table is kept for the
-        // backward one (registers for the prefetched item)
-#pragma unroll
-        for (int h = 0; h < NLEV; ++h) asm volatile("" : "+v"(pk[h]));
-      }
-      if (BWDP) {
-#pragma unroll
-        for (int h = NLEV - 1; h >= 0; --h) {
-          const unsigned int pt = pk[h];
-          if (live(pt)) {
-            const int q = pt & 0x3ff, p = (pt >> 10) & 0x1ff;
-            const C2<T> dvp = DV[p];
-            const Cpl h4 = CH[p];
-            const C2<T> b = W[q];
-            C2<T> z[3];
-#pragma unroll
-            for (int s = 0; s < 3; ++s) {
-              const unsigned int qn = unsigned(q + st[s]);
-              z[s] = W[s == 0 ? qn : min(qn, qn - unsigned(NB))];
-            }
-            C2<T> y = {T(0), T(0)};
-#pragma unroll
-            for (int s = 0; s < 3; ++s) {
-              const T c = T(h4.c[s]);
-              y.x -= c * z[s].x;
-              y.y -= c * z[s].y;
-            }
-            const C2<T> d = cmul(dvp, y);
-            W[q] = {b.x + d.x, b.y + d.y};
-          }
-          wave_sync();
-        }
-      }
-      // ---- write the item back (red forward: w; otherwise z) and the
-      // packed i-faces the other colour reads next
-      constexpr bool zp = ZP && MODE != RB_RED_FWD;
-      constexpr int zs = zp ? 2 : 1;
-      C2<T>* __restrict__ dst =
-          zp ? a.zout + (int64_t)(cu.sys >> 1) * a.zpair + (cu.sys & 1) + 2 * (int64_t)cu.tself * kBkPts
-             : a.out + o + (int64_t)cu.tself * kBkPts;
-      C2<T>* __restrict__ xfo = a.xf + (MODE == RB_RED_FWD ? 0 : a.xfhalf) +
-                                (int64_t)cu.sys * a.xfsys + (int64_t)cu.tself * kRbFaces;
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        const int p = lane + 64 * u;
-        if (!(fa < ex && fb < ey && u < ez)) continue;
-        const C2<T> zv = W[rb_box(fa, fb, u)];
-        dst[zs * p] = zv;
-        if (MODE != RB_RED_BWD && (fa == 0 || fa == TX - 1)) xfo[(fa == 0 ? 0 : 64) + fb + 8 * u] = zv;
-      }
+    for (int f = 0; f < 6; ++f) {
+      const T c = T(FC[f][lane]);
+      fv[f] = {c * fv[f].x, c * fv[f].y};
+      // (the red tiles' buffer will hold w = dinv*y)
+      if (MODE == RB_RED_BWD) fv[f] = cmul(P[face_point(f)], fv[f]);
     }
-    if (!more) break;
-    w = wn;
+  }
+  sw_order();
+  // ---- right-hand sides, with the neighbouring tiles' terms taken off
+  const C2<T> al = ccast<T>(sc.alpha);
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    C2<T> r = rv[u];
+    const int64_t pe = o + tb + lane + 64 * u;
+    if constexpr (PU) {
+      // k_pupdate's p, stored for the red tiles
+      if (sc.restart_due) {
+        a.pu_rt[pe] = r3[u];
+        r = r3[u];
+      } else {
+        r = cadd(r3[u], cmul(ccast<T>(sc.beta), csub(r, cmul(ccast<T>(sc.omg), v2[u]))));
+      }
+      a.pu_p[pe] = r;
+    } else if (FWDP && a.in2) {
+      r = csub(r, cmul(al, v2[u]));
+      if (a.sout) a.sout[pe] = r;
+    }
+    P[lane + 64 * u] = r;
+  }
+  sw_order();
+  if (HALO) {
+    // one direction after another: a tile edge lies on two faces
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+#pragma unroll
+      for (int f = 2 * s; f < 2 * s + 2; ++f) {
+        const int q = face_point(f);
+        P[q] = csub(P[q], fv[f]);
+      }
+      sw_order();
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < NU; ++u) R[u] = P[sw_point(lane, skew, u)];
+  // ---- sweeps
+  V cc[NU][3];
+  if (FWDP) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+#pragma unroll
+      for (int s = 0; s < 3; ++s) cc[u][s] = CL[s][sw_point(lane, skew, u)];
+    sw_run<false>(lane, skew, Xall[wv], [&](int u, C2<T> vi, C2<T> vj, C2<T> vk, bool act) {
+      C2<T> y = R[u];
+      y.x -= T(cc[u][0]) * vi.x;
+      y.y -= T(cc[u][0]) * vi.y;
+      y.x -= T(cc[u][1]) * vj.x;
+      y.y -= T(cc[u][1]) * vj.y;
+      y.x -= T(cc[u][2]) * vk.x;
+      y.y -= T(cc[u][2]) * vk.y;
+      const C2<T> x = cmul(D[u], y);
+      R[u] = {act ? x.x : R[u].x, act ? x.y : R[u].y};
+      return x;
+    });
+  }
+  if (BWDP) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+#pragma unroll
+      for (int s = 0; s < 3; ++s) cc[u][s] = CH[s][sw_point(lane, skew, u)];
+    sw_run<true>(lane, skew, Xall[wv], [&](int u, C2<T> vi, C2<T> vj, C2<T> vk, bool act) {
+      C2<T> y;
+      y.x = T(cc[u][0]) * vi.x;
+      y.y = T(cc[u][0]) * vi.y;
+      y.x += T(cc[u][1]) * vj.x;
+      y.y += T(cc[u][1]) * vj.y;
+      y.x += T(cc[u][2]) * vk.x;
+      y.y += T(cc[u][2]) * vk.y;
+      const C2<T> x = csub(R[u], cmul(D[u], y));
+      R[u] = {act ? x.x : R[u].x, act ? x.y : R[u].y};
+      return x;
+    });
+  }
+  // ---- back into point order and out (red forward: w; otherwise z), with
+  // the packed i-faces the other colour reads next
+  sw_order();
+#pragma unroll
+  for (int u = 0; u < NU; ++u) P[sw_point(lane, skew, u)] = R[u];
+  sw_order();
+  C2<T>* __restrict__ dst =
+      zp ? a.zout + (int64_t)(sys >> 1) * a.zpair + (sys & 1) + 2 * (int64_t)tb : a.out + o + tb;
+  C2<T>* __restrict__ xfo = a.xf + (MODE == RB_RED_FWD ? 0 : a.xfhalf) + (int64_t)sys * a.xfsys +
+                            (int64_t)tself * kRbFaces;
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    if (!(fa < ex && fb < ey && u < ez)) continue;
+    const C2<T> zv = P[lane + 64 * u];
+    dst[zs * (lane + 64 * u)] = zv;
+    if (MODE != RB_RED_BWD && (fa == 0 || fa == TX - 1)) xfo[(fa == 0 ? 0 : 64) + fb + 8 * u] = zv;
   }
 }
 

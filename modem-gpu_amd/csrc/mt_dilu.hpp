@@ -101,7 +101,7 @@ struct DiluArgs {
   // the black tiles' j- and k-faces from zout
   C2<T>* zout = nullptr;
   int64_t zpair = 0;
-  // persistent red forward sweep of the first application, when pu_r is set:
+  // red forward sweep of the first application on bricks, when pu_r is set:
   // its right-hand side is the BiCGStab p = r + beta (p - omega v) (on a
   // restart p = r and rt = r), formed from r (pu_r), the previous p (in) and
   // v (pu_v), and stored (pu_p, pu_rt) for the red tiles (the black tiles'

@@ -157,9 +157,10 @@ struct mt_ctx {
   bool sens_geom = false;
   int rb_variant = 6;           // red-black DILU: 1 persistent single-system
                                 // workgroups; 4 four systems per workgroup;
-                                // 5 the same in the lean LDS layout; 6 (on
-                                // bricks) persistent four-system workgroups
-                                // loading the next item while they sweep
+                                // 5 the same in the lean LDS layout; 6 as 5,
+                                // and on bricks (where every variant runs
+                                // k_dilu_bc) the p-update folded into the
+                                // red forward launch
   // kernel timing (mt_timing_enable): HIP events on `stream` around every
   // SpMV launch and every DILU sweep of the BiCGStab engine
   bool timing = false;
@@ -656,52 +657,47 @@ static void dilu_rb_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
   }
 }
 
-// Packed i-face buffer of the red-black sweeps for systems 0..nsys-1
-// (DiluArgs::xf); sets a.xf / a.xfsys / a.xfhalf.
-// The red-black sweeps on bricks (k_dilu_bk): the three launches of
-// dilu_rb_apply, four systems of one tile per workgroup.
-template <class T, class V>
-static void dilu_bk_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
+// The red-black sweeps on bricks (k_dilu_bc): the three launches of
+// dilu_rb_apply, up to four systems of one tile per workgroup.
+static void dilu_bk_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<float, float> a) {
   if (!a.xf) {
     ctx->err = "red-black DILU launched without its face buffer";
     return;
   }
-  constexpr int NW = 4;
+  // systems per workgroup: four share a tile's couplings; fewer active ones
+  // take smaller workgroups instead of idle waves
+  const int nw = a.nact >= 3 ? 4 : a.nact;
   for (int step = 0; step < 3; ++step) {
     const int L = (step == 1) ? 1 : 0;
     if (L >= tp.nlev) continue;
     a.tiles = tp.tiles + tp.lvl_off[L];
     a.ntiles = tp.lvl_off[L + 1] - tp.lvl_off[L];
     if (a.ntiles == 0) continue;
-    const int64_t nwork = int64_t(a.ntiles) * ((a.nact + NW - 1) / NW);
+    const int64_t nwork = int64_t(a.ntiles) * ((a.nact + nw - 1) / nw);
     const int g = int(8 * ((nwork + 7) / 8));
-    // the result pair-interleaved (zout: FP32 inner solves with paired x)
-    auto launch = [&](auto zp) {
+    // zp: the result pair-interleaved (zout: FP32 inner solves with paired x)
+    auto launch = [&](auto nwc, auto zp) {
+      constexpr int NW = decltype(nwc)::value;
       constexpr bool ZP = decltype(zp)::value;
-      if (ctx->rb_variant == 6) {
-        // persistent: three workgroups per CU (their LDS), a multiple of 8 XCDs
-        const int gp = std::min(g, std::max(8, ctx->num_cu * 3 / 8 * 8));
-        if (step == 0 && a.pu_r)   // (the p-update folded into the red forward sweep)
-          k_dilu_bkp<T, V, RB_RED_FWD, NW, ZP, true><<<gp, 64 * NW, 0, ctx->stream>>>(a, tp.shape);
-        else if (step == 0) k_dilu_bkp<T, V, RB_RED_FWD, NW, ZP><<<gp, 64 * NW, 0, ctx->stream>>>(a, tp.shape);
-        else if (step == 1) k_dilu_bkp<T, V, RB_BLACK_FB, NW, ZP><<<gp, 64 * NW, 0, ctx->stream>>>(a, tp.shape);
-        else k_dilu_bkp<T, V, RB_RED_BWD, NW, ZP><<<gp, 64 * NW, 0, ctx->stream>>>(a, tp.shape);
-        return;
-      }
-      if (step == 0) k_dilu_bk<T, V, RB_RED_FWD, NW, ZP><<<g, 64 * NW, 0, ctx->stream>>>(a, tp.shape);
-      else if (step == 1) k_dilu_bk<T, V, RB_BLACK_FB, NW, ZP><<<g, 64 * NW, 0, ctx->stream>>>(a, tp.shape);
-      else k_dilu_bk<T, V, RB_RED_BWD, NW, ZP><<<g, 64 * NW, 0, ctx->stream>>>(a, tp.shape);
+      const hipStream_t st = ctx->stream;
+      if (step == 0 && a.pu_r)   // (the p-update folded into the red forward sweep)
+        k_dilu_bc<float, float, RB_RED_FWD, NW, ZP, true><<<g, 64 * NW, 0, st>>>(a);
+      else if (step == 0) k_dilu_bc<float, float, RB_RED_FWD, NW, ZP><<<g, 64 * NW, 0, st>>>(a);
+      else if (step == 1) k_dilu_bc<float, float, RB_BLACK_FB, NW, ZP><<<g, 64 * NW, 0, st>>>(a);
+      else k_dilu_bc<float, float, RB_RED_BWD, NW, ZP><<<g, 64 * NW, 0, st>>>(a);
     };
-    if constexpr (sizeof(T) == 4) {
-      if (a.zout) {
-        launch(std::true_type());
-        continue;
-      }
-    }
-    launch(std::false_type());
+    auto launch_nw = [&](auto zp) {
+      if (nw == 4) launch(Comp<4>(), zp);
+      else if (nw == 2) launch(Comp<2>(), zp);
+      else launch(Comp<1>(), zp);
+    };
+    if (a.zout) launch_nw(std::true_type());
+    else launch_nw(std::false_type());
   }
 }
 
+// Packed i-face buffer of the red-black sweeps for systems 0..nsys-1
+// (DiluArgs::xf); sets a.xf / a.xfsys / a.xfhalf.
 template <class T, class V>
 static int rb_faces(mt_ctx* ctx, int nsys, DiluArgs<T, V>& a) {
   const TilePlan& tp = ctx->tiles_rb;
@@ -859,8 +855,8 @@ struct Engine {
     d.xfsys = xfsys;
     d.xfhalf = xfhalf;
     const int e0 = ctx->timing ? trec() : -1;
-    if (brick) dilu_bk_apply<T, V>(ctx, tp, d);
-    else apply_pc(d);
+    if (!brick) apply_pc(d);
+    else if constexpr (sizeof(T) == 4) dilu_bk_apply(ctx, tp, d);
     if (ctx->timing) tpairs.push_back({MT_KT_PRECOND, e0, trec()});
   }
   // the SpMV and its dot partials; returns the partial count per system
@@ -905,7 +901,7 @@ struct Engine {
   }
 
   // the p-update folded into the first application's red forward sweep:
-  // inner solves on bricks with the persistent red-black sweeps
+  // inner solves on bricks
   bool pfold() const {
     return brick && a.fused && a.pc == PCK_DILU_RB && ctx->rb_variant == 6 && ctx->tiles_rb.nlev == 2;
   }
@@ -1790,7 +1786,7 @@ int mt_precond_apply(mt_ctx* ctx, double omega, int precond, const mt_zdouble* x
 
 
 // The inner solves' brick kernels on one vector: y = A x (what 0, k_spmv_bt)
-// or y = M^-1 x (what 1, k_dilu_bk with the red-black DILU of A(omega)), of A
+// or y = M^-1 x (what 1, k_dilu_bc with the red-black DILU of A(omega)), of A
 // or of A^T, in FP32 on bricks; x and y in EDGEi order, FP64.
 int mt_inner_apply(mt_ctx* ctx, double omega, int what, int transpose, const mt_zdouble* x,
                    mt_zdouble* y) {
@@ -1850,7 +1846,7 @@ int mt_inner_apply(mt_ctx* ctx, double omega, int what, int transpose, const mt_
     DiluArgs<float, float> d = dilu_args<float, float>(ctx->tiles_rb, ctx->bk.slots[tr ? 1 : 0], nB, nB,
                                                        d_act, 1, d_sc, xb, yb, db, ST_RUN);
     if ((rc = rb_faces(ctx, 1, d))) return rc;
-    dilu_bk_apply<float, float>(ctx, ctx->tiles_rb, d);
+    dilu_bk_apply(ctx, ctx->tiles_rb, d);
   }
   k_bk_from_brick<<<2048, BS, 0, ctx->stream>>>(d_act, 1, ctx->bk.bmap, nB, nE, yb, yn);
   MT_HIP_CHECK(ctx, hipMemsetAsync(dy, 0, sizeof(Z) * g.nE, ctx->stream));
@@ -2386,7 +2382,7 @@ int mt_bench_precond(mt_ctx* ctx, int nsys, int precision, int precond, int reps
     if (precond == MT_PC_DILU_RB && (r2 = rb_faces(ctx, nsys, d))) return r2;
     auto apply = [&]() {
       if (bricks) {
-        dilu_bk_apply<T, T>(ctx, tp, d);
+        if constexpr (sizeof(T) == 4) dilu_bk_apply(ctx, tp, d);
       } else if (precond == MT_PC_DILU_RB) {
         dilu_rb_apply<T, T>(ctx, tp, d);
       } else {

@@ -179,3 +179,21 @@ def test_brick_solves_match_all_edge_layout(gpu_ctx, transpose):
             assert rel(X[s], xo) <= 1e-7, bricks
         nb, na = res[True][1][s]["niter"], res[False][1][s]["niter"]
         assert abs(nb - na) <= 0.25 * max(nb, na) + 10, (nb, na)
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(9, 8, 8), (8, 17, 10), (16, 9, 24), (5, 3, 4)])
+def test_brick_dilu_tile_edges(gpu_ctx, nx, ny, nz):
+    """The register sweeps at the edges of the tiles: grids whose lattices
+    fill their last tile with one, seven or all eight layers, or fit one tile.
+    Against the FP64 apply in the same ordering; FP32 sweeps accumulate over at
+    most 22 dependent points per tile and three tile levels, 2e-5 as above."""
+    print(f"case brick dilu edges {nx}x{ny}x{nz}", flush=True)
+    nza = max(1, nz // 4)
+    dx, dy, dz, nza, lc = small_problem(47, nx=nx, ny=ny, nzAir=nza, nzEarth=nz - nza)
+    gpu_ctx.assemble(dx, dy, dz, nza, lc)
+    rng = np.random.default_rng(7)
+    x = rng.standard_normal(gpu_ctx.n_int) + 1j * rng.standard_normal(gpu_ctx.n_int)
+    for f in (1e-2, 5.0):
+        w = 2 * np.pi * f
+        z = gpu_ctx.inner_apply(w, x, what=1)
+        assert rel(z, gpu_ctx.precond_apply(w, x, mtsp2.PC_DILU_RB)) <= 2e-5, f
