@@ -12,10 +12,11 @@
 // on both sides of the diagonal.
 //
 // k_bc_te1d solves every 1-D column, one thread each.  k_bc_te2d solves one
-// slice per workgroup: the band's active (nz x nz) window stays in LDS as a
-// circular buffer over rows and columns, the right-hand side is eliminated
-// as the factorisation proceeds, the rows of U go to a per-workgroup scratch
-// in HBM, and one wave back-substitutes from staged chunks of U.
+// slice per workgroup: the band's active (nz x nz) window stays in registers
+// as a circular buffer over rows and columns, the right-hand side is
+// eliminated as the factorisation proceeds, the rows of U go to a
+// per-workgroup scratch in HBM, and one wave back-substitutes from staged
+// chunks of U.
 //
 // Every complex product and quotient is formed as the reference's BLAS and
 // LAPACK form it (textbook products, C99 Annex G division as __divdc3 does
@@ -30,10 +31,16 @@
 #include "mt_device.hpp"
 #include "mt_dilu.hpp"
 #include "mt_internal.h"
+#include "mt_sweep.hpp"
 
 namespace mt {
 
-constexpr int kBcChunk = 32;   // factorisation steps per staged chunk of entering coefficients
+constexpr int kBcChunk = 128;  // factorisation steps per staged chunk of entering coefficients
+constexpr int kBcBack = 16;    // back-substitution steps per staged chunk of U
+
+// A node's diagonal, right-hand side and couplings to the next node in z and
+// in the horizontal.
+struct BcCoef { double2 d, r; double a2, a3; };
 
 struct BcArgs {
   int nx, ny, nz, nza;          // 3-D grid; nz counts the air layers
@@ -49,11 +56,18 @@ struct BcArgs {
   int mmbMax;                   // boundary vector length per item (1-based, index 0 unused)
   double2* exb;                 // [nitem][mmbMax] boundary values of each slice (EXB)
   double2* side;                // [nitem][2][nz][2] factors of the two side columns
-  double2* ucol;                // per workgroup [nmax][nz]: ucol[j-1][o] = U(j-o, j)
-  double2* yx;                  // per workgroup [nmax]: eliminated rhs, then the solution
-  int64_t uStride, yStride;
   int* flag;                    // [nitem] 1 if the reference's LU would pivot (or a zero pivot)
   double2* e;                   // [nsys][nE] out: E0 inside, the boundary conditions outside
+};
+
+// Per-workgroup scratch of k_bc_te2d: urow [nmax][M], urow[j-1][c] = U(j, j+c) (M >= nz slots);
+// yx [nmax], the eliminated rhs, then the solution; coef [nmax], the slice's
+// matrix and rhs by node.
+struct BcScratch {
+  double2 *urow, *yx;
+  BcCoef* coef;
+  int64_t nmax;
+  int nz, nitem;
 };
 
 struct BcSlice {
@@ -85,21 +99,48 @@ __device__ __forceinline__ double2 bz_mul(double2 a, double2 b) {
 }
 
 // complex quotient, C99 Annex G (G.5.1) for finite operands: the divisor
-// scaled by 2^-logb(max(|c|, |d|))
-__device__ __forceinline__ double2 bz_div(double2 n, double2 d) {
+// scaled by 2^-logb(max(|c|, |d|)).  In two steps, so that what depends on the
+// divisor alone can be formed ahead: den = |scaled divisor|^2 lies in [1, 8)
+// and inv is 1/den to the last bit or so; a quotient n/den is n*inv with one
+// correction from its exact remainder, which is the correctly rounded one (the
+// steps of the hardware's own division without its rescaling) while neither
+// n nor the remainder leaves the normal range; else n/den is divided as such.
+struct BzDen { double c, e, den, inv; int il; };
+__device__ __forceinline__ BzDen bz_den(double2 d) {
 #pragma clang fp contract(off)
-  const double a = n.x, b = n.y;
-  double c = d.x, e = d.y;
-  int il = 0;
-  const double lw = logb(fmax(fabs(c), fabs(e)));
-  if (isfinite(lw)) {
-    il = int(lw);
-    c = scalbn(c, -il);
-    e = scalbn(e, -il);
+  BzDen q;
+  q.c = d.x;
+  q.e = d.y;
+  q.il = 0;
+  const double mx = fmax(fabs(q.c), fabs(q.e));
+  if (mx > 0.0 && mx < HUGE_VAL) {   // logb(mx) is finite
+    q.il = __builtin_amdgcn_frexp_exp(mx) - 1;
+    q.c = scalbn(q.c, -q.il);
+    q.e = scalbn(q.e, -q.il);
   }
-  const double den = c * c + e * e;
-  return make_double2(scalbn((a * c + b * e) / den, -il), scalbn((b * c - a * e) / den, -il));
+  q.den = q.c * q.c + q.e * q.e;
+  double r = __builtin_amdgcn_rcp(q.den);
+  r = __builtin_fma(r, __builtin_fma(-q.den, r, 1.0), r);
+  q.inv = __builtin_fma(r, __builtin_fma(-q.den, r, 1.0), r);
+  return q;
 }
+__device__ __forceinline__ double2 bz_div(double2 n, const BzDen& q) {
+#pragma clang fp contract(off)
+  const double nx = n.x * q.c + n.y * q.e, ny = n.y * q.c - n.x * q.e;
+  double x = nx * q.inv, y = ny * q.inv;
+  x = __builtin_fma(__builtin_fma(-q.den, x, nx), q.inv, x);
+  y = __builtin_fma(__builtin_fma(-q.den, y, ny), q.inv, y);
+  // 2^-900 .. 2^900, or zero over a den in its range
+  const double lo = 0x1p-900, hi = 0x1p900, ax = fabs(nx), ay = fabs(ny);
+  const bool ok = q.den >= 1.0 && q.den < 8.0 && (ax == 0.0 || ax > lo) && ax < hi &&
+                  (ay == 0.0 || ay > lo) && ay < hi;
+  if (!ok) {
+    x = nx / q.den;
+    y = ny / q.den;
+  }
+  return make_double2(scalbn(x, -q.il), scalbn(y, -q.il));
+}
+__device__ __forceinline__ double2 bz_div(double2 n, double2 d) { return bz_div(n, bz_den(d)); }
 
 __device__ __forceinline__ bool bz_nz(double2 v) { return v.x != 0.0 || v.y != 0.0; }
 __device__ __forceinline__ double bz_abs1(double2 v) { return fabs(v.x) + fabs(v.y); }
@@ -267,244 +308,374 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-__host__ __device__ inline size_t bc_lds_bytes(int nz) {
+// Largest nz the slices are taken at (an (nz x nz) window of complex doubles
+// and its staging within 160 KB).
+__host__ __device__ inline size_t bc_window_bytes(int nz) {
   const size_t B1 = size_t(nz);
-  return (B1 * B1 + B1 + 2 * kBcChunk + 1) * sizeof(double2) + 2 * kBcChunk * sizeof(double);
+  return (B1 * B1 + B1 + 65) * sizeof(double2) + 64 * sizeof(double);
 }
 
-// One slice per workgroup, persistent over the items.  Window slot of node r
-// is r mod nz (nz = bandwidth + 1); W[cs*nz + rs] holds A(r, c).
-__global__ __launch_bounds__(256) void k_bc_te2d(BcArgs a) {
-#pragma clang fp contract(off)
-  extern __shared__ double2 lds[];
-  __shared__ int sflag;
-  const int b = a.nz - 1, B1 = a.nz;
-  double2* W = lds;
-  double2* Bv = W + B1 * B1;
-  double2* Ed = Bv + B1;
-  double2* Er = Ed + kBcChunk;
-  double* Ea2 = reinterpret_cast<double*>(Er + kBcChunk);
-  double* Ea3 = Ea2 + kBcChunk;
-  double2* Rp = reinterpret_cast<double2*>(Ea3 + kBcChunk);   // 1 / next pivot
-  const int tid = threadIdx.x, nt = blockDim.x;
-  double2* U = a.ucol + (int64_t)blockIdx.x * a.uStride;
-  double2* Y = a.yx + (int64_t)blockIdx.x * a.yStride;
-  // (selects below are written as assignments: a ?: between a local double2
-  // and a memory operand becomes a select of addresses, which keeps the
-  // local in scratch)
+// The arguments as if met for the first time: what one phase of a slice reads
+// of them is not kept in registers over the others.
+__device__ __forceinline__ const BcArgs* bc_reload(const BcArgs* p) {
+  asm volatile("" : "+s"(p));
+  return p;
+}
 
-  for (int it = blockIdx.x; it < a.nitem; it += gridDim.x) {
-    const BcSlice S = bc_slice(a, it);
-    const int Ny = S.nh, n = (Ny - 1) * b;
-    const double2* exb = a.exb + (int64_t)it * a.mmbMax;
+// v of a wave's lane `l` (uniform)
+__device__ __forceinline__ double bc_lane(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+__device__ __forceinline__ double2 bc_lane(double2 v, int l) {
+  return make_double2(bc_lane(v.x, l), bc_lane(v.y, l));
+}
+
+// One slice per workgroup of TG x TG threads, persistent over the items.
+//
+// The window: node r has slot r mod M, M = TG*R >= nz (the nodes j .. j+nz-1
+// of step j hold distinct slots); thread (tr, tc) keeps A(r, c) of the R x R
+// slots (tr + TG*ii, tc + TG*jj) in registers, 0 where the slots hold no node.
+// A step j is
+//   export  (at the end of step j-1): the wave that holds column j forms the
+//           multipliers l = A(:, j) (1/p) and the rhs update, the threads of
+//           row j store U(j, :); both go to LDS vectors by slot (two sets,
+//           alternating) and the slot's row and column become zero;
+//   barrier;
+//   the entering node's coefficients are placed, then every thread updates
+//   its R x R entries with the R multipliers and R row values it reads.
+// What bounds it: with many slices the issue of FP64 products and sums
+// without contraction, eight per entry and step (three slices per CU at nz =
+// 70: 3,530 cycles a step, 3 x 1,200 of issue), and the rounds (1,600 slices of
+// 100 x 70 on 768 resident workgroups leave 64 for a third); with few the
+// chain of a step (1/p 440 cycles, multipliers 450, update 570 at nz = 35).
+// With the window in LDS a step moved 290 KB there and took two barriers:
+// 1,600 slices of 100 x 70 97 ms, now 43; 78 of 45 x 35 3.4 ms, now 2.1.
+template <int TG, int R>
+struct BcShape {
+  static constexpr int M = TG * R, NT = TG * TG;
+  // waves per SIMD the register window leaves room for
+  static constexpr int WAVES = R <= 4 ? 4 : (R == 5 ? 3 : (R == 6 ? 2 : 1));
+};
+
+__host__ __device__ inline size_t bc_back_bytes(int nz) {
+  return (size_t(kBcBack) * nz + 2 * kBcBack) * sizeof(double2) + kBcBack * sizeof(BzDen);
+}
+
+template <int TG, int R>
+__global__ __launch_bounds__(TG * TG, (BcShape<TG, R>::WAVES)) void k_bc_te2d(const BcArgs* __restrict__ ap, BcScratch w) {
+#pragma clang fp contract(off)
+  constexpr int M = BcShape<TG, R>::M, NT = BcShape<TG, R>::NT;
+  static_assert(NT % 64 == 0 && 64 % TG == 0, "a column's threads lie in one wave");
+  extern __shared__ double2 lds[];   // back substitution: kBcBack columns of U, as many rhs entries
+  __shared__ double2 Lv[2][M], Uv[2][M], Pv[2], Bv[M];
+  __shared__ double2 Ed[2][kBcChunk], Er[2][kBcChunk];
+  __shared__ double Ea2[2][kBcChunk], Ea3[2][kBcChunk];
+  __shared__ int sflag;
+  const int b = w.nz - 1, B1 = w.nz;
+  const int tid = threadIdx.x, tr = tid % TG, tc = tid / TG, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  double2* __restrict__ U = w.urow + (int64_t)blockIdx.x * w.nmax * M;
+  double2* __restrict__ Y = w.yx + (int64_t)blockIdx.x * w.nmax;
+  BcCoef* __restrict__ C = w.coef + (int64_t)blockIdx.x * w.nmax;
+
+  for (int it = blockIdx.x; it < w.nitem; it += gridDim.x) {
     if (tid == 0) sflag = 0;
-    int myflag = 0;
-    for (int q = tid; q < B1 * B1; q += nt) W[q] = make_double2(0.0, 0.0);
-    __syncthreads();
-    // the window of step 1: nodes 1..min(b, n)
-    const int n0 = min(b, n);
-    for (int r = 1 + tid; r <= n0; r += nt) {
-      int iy, iz;
-      bc_node(b, r, iy, iz);
-      W[(r % B1) * B1 + r % B1] = bc_diag(a, S, iy, iz);
-      if (r + 1 <= n0) {
-        const double2 v = make_double2(bc_a2(a, S, iy, iz), 0.0);
-        W[((r + 1) % B1) * B1 + r % B1] = v;
-        W[(r % B1) * B1 + (r + 1) % B1] = v;
+    int n;
+    {
+      const BcArgs a = *bc_reload(ap);
+      const BcSlice S = bc_slice(a, it);
+      const double2* exb = a.exb + (int64_t)it * a.mmbMax;
+      n = __builtin_amdgcn_readfirstlane((S.nh - 1) * b);
+      for (int q = 1 + tid; q <= n; q += NT) {
+        int iy, iz;
+        bc_node(b, q, iy, iz);
+        BcCoef v;
+        v.d = bc_diag(a, S, iy, iz);
+        v.r = bc_rhs(a, S, exb, iy, iz);
+        v.a2 = bc_a2(a, S, iy, iz);
+        v.a3 = bc_a3(a, S, iy, iz);
+        C[q - 1] = v;
       }
-      Bv[r % B1] = bc_rhs(a, S, exb, iy, iz);
     }
-    for (int j = 1; j <= n; ++j) {
-      const int cs = (j - 1) % kBcChunk;
-      if (cs == 0) {
-        // coefficients entering at steps j .. j+kBcChunk-1: node q = step+b
-        // (diagonal, rhs, z-coupling to q-1) and the horizontal coupling of the step's own node
-        for (int s = tid; s < kBcChunk; s += nt) {
-          const int jj = j + s, q = jj + b;
-          int iy, iz;
-          if (q <= n) {
-            bc_node(b, q, iy, iz);
-            Ed[s] = bc_diag(a, S, iy, iz);
-            Er[s] = bc_rhs(a, S, exb, iy, iz);
-            bc_node(b, q - 1, iy, iz);
-            Ea2[s] = bc_a2(a, S, iy, iz);
-          }
-          if (jj <= n) {
-            bc_node(b, jj, iy, iz);
-            Ea3[s] = bc_a3(a, S, iy, iz);
+    __syncthreads();
+    // the window of step 1: nodes 1 .. b (n >= b) in the slots of their numbers
+    double Ax[R][R], Ay[R][R];
+#pragma unroll
+    for (int ii = 0; ii < R; ++ii)
+#pragma unroll
+      for (int jj = 0; jj < R; ++jj) {
+        const int r = tr + TG * ii, c = tc + TG * jj, lo = min(r, c);
+        Ax[ii][jj] = Ay[ii][jj] = 0.0;
+        if (lo >= 1 && max(r, c) <= b) {
+          if (r == c) {
+            Ax[ii][jj] = C[lo - 1].d.x;
+            Ay[ii][jj] = C[lo - 1].d.y;
+          } else if (r - c == 1 || c - r == 1) {
+            Ax[ii][jj] = C[lo - 1].a2;
           }
         }
       }
-      lds_barrier();
-      const int m = min(b, n - j), sj = j % B1, q = j + b, sq = q % B1;
-      const double2 p = W[sj * B1 + sj];
-      const double2 yv = Bv[sj];
-      const double2 a3j = make_double2(Ea3[cs], 0.0);
-      if (tid >= 1 && tid <= m) {
-        // column j of L: l_i = A(j+i, j) / p, the rhs update, the pivot test
-        const int i = tid;
-        int si = sj + i;
-        if (si >= B1) si -= B1;
-        double2 ai = a3j;
-        if (i != b) ai = W[sj * B1 + si];
-        if (!(bz_abs1(ai) <= bz_abs1(p))) myflag = 1;
-        double2 r;
-        if (j == 1) r = bz_div(make_double2(1.0, 0.0), p);
-        else r = Rp[0];
-        const double2 l = bz_mul(r, ai);
-        W[sj * B1 + si] = l;
-        double2 base;
-        if (i == b) base = Er[cs];
-        else base = Bv[si];
-        if (bz_nz(yv)) {
-          const double2 u = bz_mul(l, yv);
-          base = make_double2(base.x - u.x, base.y - u.y);
+    for (int q = tid; q < M; q += NT) {
+      double2 v = make_double2(0.0, 0.0);
+      if (q >= 1 && q <= b) v = C[q - 1].r;
+      Bv[q] = v;
+    }
+    // the coefficients of steps j0 .. j0+kBcChunk-1: node step+b's diagonal and
+    // rhs, its z-coupling to the node before, the step's own horizontal coupling
+    auto stage = [&](int j0, int buf) {
+      for (int t = tid; t < kBcChunk; t += NT) {
+        const int jj = j0 + t, q = jj + b;
+        if (q <= n) {
+          Ed[buf][t] = C[q - 1].d;
+          Er[buf][t] = C[q - 1].r;
+          Ea2[buf][t] = C[q - 2].a2;
         }
-        Bv[si] = base;
+        if (jj <= n) Ea3[buf][t] = C[jj - 1].a3;
       }
-      if (tid <= m) {
-        // row j of U, by column into the scratch
-        const int c = tid;
-        int sc = sj + c;
-        if (sc >= B1) sc -= B1;
-        double2 u;
-        if (c == 0) u = p;
-        else if (c == b) u = a3j;
-        else u = W[sc * B1 + sj];
-        U[(int64_t)(j + c - 1) * B1 + c] = u;
-      }
-      if (tid == 0) {
-        Y[j - 1] = yv;
-        if (!bz_nz(p)) myflag = 1;
-      }
-      if (q <= n) {
-        if (tid <= b) {
-          // the entering column q: rows j..q
-          const int r = j + tid;
-          double2 v = make_double2(0.0, 0.0);
-          if (r == j) v = a3j;
-          else if (r == q - 1) v = make_double2(Ea2[cs], 0.0);
-          else if (r == q) v = Ed[cs];
-          W[sq * B1 + r % B1] = v;
-        }
-        if (tid >= 1 && tid <= b - 1) {
-          // the entering row q: columns j+1..q-1
-          const int c = j + tid;
-          W[(c % B1) * B1 + sq] = make_double2(c == q - 1 ? Ea2[cs] : 0.0, 0.0);
-        }
-      }
-      lds_barrier();
-      // rank-1 update of the trailing m x m block (ZGERU order per entry):
-      // thread (g, i) owns rows i and i + mh and every G-th column from 1+g,
-      // so each U-row value it reads serves two entries and its multipliers
-      // are read once; four columns are in flight at a time.  The owner of
-      // the next pivot (row 1, column 1: thread 0) also forms its reciprocal
-      // for the next step.
-      if (m > 0) {
-        const int mh = (m + 1) / 2, G = nt / mh, g = tid / mh, i = 1 + tid % mh, i2 = i + mh;
-        if (g < G) {
-          const bool two = i2 <= m;
-          int si = sj + i, si2 = sj + i2;
-          if (si >= B1) si -= B1;
-          if (si2 >= B1) si2 -= B1;
-          const double2 l = W[sj * B1 + si];
-          double2 l2 = make_double2(0.0, 0.0);
-          if (two) l2 = W[sj * B1 + si2];
-          int c = 1 + g;
-          for (; c + 3 * G <= m; c += 4 * G) {
-            int sc[4];
-            double2 y[4], w[4], w2[4];
+    };
+    stage(1, 0);
+    __syncthreads();
+
+    // (the window is in registers here: with its loads still pending at the
+    // loop, every step would wait for its own stores of U)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              sc[k] = sj + c + k * G;
-              if (sc[k] >= B1) sc[k] -= B1;
-              y[k] = W[sc[k] * B1 + sj];
-              w[k] = W[sc[k] * B1 + si];
-              if (two) w2[k] = W[sc[k] * B1 + si2];
-            }
+    for (int ii = 0; ii < R; ++ii)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const double2 u = bz_mul(l, y[k]);
-              w[k] = make_double2(w[k].x - u.x, w[k].y - u.y);
-              W[sc[k] * B1 + si] = w[k];
-              if (two) {
-                const double2 u2 = bz_mul(l2, y[k]);
-                W[sc[k] * B1 + si2] = make_double2(w2[k].x - u2.x, w2[k].y - u2.y);
+      for (int jj = 0; jj < R; ++jj) asm volatile("" : "+v"(Ax[ii][jj]), "+v"(Ay[ii][jj]));
+    // the steps, slot by slot of the pivot: sj = ts + TG*ip with ip a constant
+    int j = 1, ts = 1 % TG, sj = 1, sq = (1 + b) % M;
+    // step jn's entering coefficients: read a step ahead where there are
+    // registers for them (R = 5 spills with eight more)
+    constexpr bool AHEAD = R <= 4;
+    double2 ed;
+    double e2, e3;
+    auto entering = [&](int jn) {
+      const int c1 = (jn - 1) % kBcChunk, b1 = ((jn - 1) / kBcChunk) & 1;
+      ed = Ed[b1][c1];
+      e2 = Ea2[b1][c1];
+      e3 = Ea3[b1][c1];
+    };
+    entering(1);
+    while (j <= n) {
+#pragma unroll
+      for (int ip = 0; ip < R; ++ip) {
+        for (; ts < TG && j <= n; ++ts, ++j) {
+          // (opaque: nothing a step derives from the grid position is kept in
+          // registers over the steps.  A spilled register's reload would wait
+          // for the step's stores of U)
+          int r0 = tr, c0 = tc;
+          asm volatile("" : "+v"(r0), "+v"(c0));
+          const int par = j & 1, cs = (j - 1) % kBcChunk, buf = ((j - 1) / kBcChunk) & 1;
+          const bool own = wave == (ts * TG) >> 6;   // this wave's threads c0 == ts hold column j
+          if (j + b <= n) {
+            if constexpr (!AHEAD) entering(j);
+            // node q = j+b enters: its diagonal, its couplings to q-1 and to j
+            // (slot sq, empty until here)
+            const int iq = sq / TG, tq = sq % TG, t1 = (tq + TG - 1) % TG;
+            const bool wq = wave == (tq * TG) >> 6;
+            if (own || wq || wave == (t1 * TG) >> 6) {
+#pragma unroll
+              for (int ii = 0; ii < R; ++ii) {
+                if (ii != iq) continue;   // uniform
+                const int im = (ii + R - 1) % R;
+                if (wq && c0 == tq) {
+                  if (r0 == tq) {
+                    Ax[ii][ii] = ed.x;
+                    Ay[ii][ii] = ed.y;
+                  }
+                  if (r0 == t1) {
+                    if (tq > 0) Ax[ii][ii] = e2;
+                    else Ax[im][ii] = e2;
+                  }
+                  if (r0 == ts) Ax[ip][ii] = e3;
+                }
+                if (c0 == t1 && r0 == tq) {
+                  if (tq > 0) Ax[ii][ii] = e2;
+                  else Ax[ii][im] = e2;
+                }
+                if (own && c0 == ts && r0 == tq) Ax[ii][ip] = e3;
               }
             }
-            if (tid == 0 && c == 1) Rp[0] = bz_div(make_double2(1.0, 0.0), w[0]);
           }
-          for (; c <= m; c += G) {
-            int sc = sj + c;
-            if (sc >= B1) sc -= B1;
-            const double2 yv2 = W[sc * B1 + sj];
-            const double2 u = bz_mul(l, yv2);
-            const double2 w0 = W[sc * B1 + si];
-            const double2 wn = make_double2(w0.x - u.x, w0.y - u.y);
-            W[sc * B1 + si] = wn;
-            if (two) {
-              const double2 u2 = bz_mul(l2, yv2);
-              const double2 w1 = W[sc * B1 + si2];
-              W[sc * B1 + si2] = make_double2(w1.x - u2.x, w1.y - u2.y);
+          if (own) {
+            __builtin_amdgcn_s_setprio(1);   // the others wait for this wave
+            // thread r0 == c0 == ts holds the pivot
+            const double2 p =
+                bc_lane(make_double2(Ax[ip][ip], Ay[ip][ip]), (ts * TG + ts) & 63);
+            const double2 rp = bz_div(make_double2(1.0, 0.0), p);
+            if (c0 == ts) {
+              const double pa = bz_abs1(p);
+              bool bad = !bz_nz(p);
+#pragma unroll
+              for (int ii = 0; ii < R; ++ii) {
+                const double2 v = make_double2(Ax[ii][ip], Ay[ii][ip]);
+                const bool piv = ii == ip && r0 == ts;   // (multiplier 0 in the pivot's own slot)
+                const double2 l = bz_mul(rp, v);
+                Lv[par][r0 + TG * ii] = make_double2(piv ? 0.0 : l.x, piv ? 0.0 : l.y);
+                if (piv) Pv[par] = v;
+                bad |= !(bz_abs1(v) <= pa);
+                Ax[ii][ip] = Ay[ii][ip] = 0.0;
+              }
+              if (bad) sflag = 1;
             }
-            if (tid == 0 && c == 1) Rp[0] = bz_div(make_double2(1.0, 0.0), wn);
+            __builtin_amdgcn_s_setprio(0);
           }
+          if (r0 == ts) {
+#pragma unroll
+            for (int jj = 0; jj < R; ++jj) {
+              // (the pivot's own slot: zero, as above or by the column's threads)
+              const bool piv = jj == ip && c0 == ts;
+              Uv[par][c0 + TG * jj] = make_double2(piv ? 0.0 : Ax[ip][jj], piv ? 0.0 : Ay[ip][jj]);
+              Ax[ip][jj] = Ay[ip][jj] = 0.0;
+            }
+          }
+          lds_barrier();
+          if constexpr (AHEAD) entering(j + 1);
+          double2 l[R];
+#pragma unroll
+          for (int ii = 0; ii < R; ++ii) l[ii] = Lv[par][r0 + TG * ii];
+          // (a column's row value is read one column ahead, not all at once:
+          // registers)
+          double2 u = Uv[par][c0];
+#pragma unroll
+          for (int jj = 0; jj < R; ++jj) {
+            const double2 un = Uv[par][c0 + TG * (jj + 1 < R ? jj + 1 : jj)];
+#pragma unroll
+            for (int ii = 0; ii < R; ++ii) {
+              const double2 t = bz_mul(l[ii], u);
+              Ax[ii][jj] -= t.x;
+              Ay[ii][jj] -= t.y;
+            }
+            u = un;
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          // row j of U, entry c (node j+c, slot s = sj + c mod M, zero in empty
+          // slots), and the rhs of row j+c: by threads of the waves that do not
+          // hold the next columns
+          const int t = (tid - 64 * ((ts * TG >> 6) + 2)) & (NT - 1);
+          if (t < M) {
+            int s = sj + t;
+            if (s >= M) s -= M;
+            const double2 yv = Bv[sj], ls = Lv[par][s];
+            double2 u = Uv[par][s], base = Bv[s];
+            if (s == sq && j + b <= n) base = Er[buf][cs];
+            if (t == 0) {
+              u = Pv[par];
+              Y[j - 1] = yv;
+            } else {
+              if (bz_nz(yv)) {
+                const double2 d = bz_mul(ls, yv);
+                base = make_double2(base.x - d.x, base.y - d.y);
+              }
+              Bv[s] = base;
+            }
+            U[(int64_t)(j - 1) * M + t] = u;
+          }
+          // (read from step j0+kBcChunk on, barriers later)
+          if (cs == 0 && j + kBcChunk <= n) stage(j + kBcChunk, buf ^ 1);
+          if (++sj == M) sj = 0;
+          if (++sq == M) sq = 0;
         }
+        if (ts == TG) ts = 0;
       }
     }
-    if (myflag) atomicOr(&sflag, 1);
     __syncthreads();
-    if (tid == 0) a.flag[it] = sflag;
+    if (tid == 0) ap->flag[it] = sflag;
+
     // back substitution with U (ZTBSV order): x_j = y_j / U(j,j), then
-    // y_{j-o} -= x_j U(j-o, j) for o = 1..b; the y window is Bv
-    for (int r = max(1, n - b) + tid; r <= n; r += nt) Bv[r % B1] = Y[r - 1];
-    for (int j1 = n; j1 >= 1; j1 -= b) {
-      const int j0 = max(1, j1 - b + 1), cnt = j1 - j0 + 1;
-      __syncthreads();
-      // stage U columns j0..j1 into W[(jj-j0)*B1 + o] and the entering y_{jj-b} into W[b*B1 + jj-j0]
-      for (int e = tid; e < cnt * B1; e += nt) {
-        const int jj = j0 + e / B1, o = e % B1;
-        double2 v = make_double2(0.0, 0.0);
-        if (o <= jj - 1) v = U[(int64_t)(jj - 1) * B1 + o];
-        W[(jj - j0) * B1 + o] = v;
+    // y_{j-o} -= x_j U(j-o, j) for o = 1..b.  Wave 0 keeps the open rows, row
+    // i in lane i mod 64 (ra the lane's highest open row, ya its value, yb row
+    // ra-64's); the columns of U are staged by chunk, the next chunk's loads
+    // in flight meanwhile.
+    double2* SU = lds;                   // [k][o] = U(j-o, j), j = j0+k
+    double2* SY = lds + kBcBack * B1;    // [k] = y of row j-128
+    double2* SX = SY + kBcBack;          // [k] = x_j
+    BzDen* SD = reinterpret_cast<BzDen*>(SX + kBcBack);   // [k]: U(j,j) as a divisor
+    constexpr int NE = ((kBcBack + M) * kBcBack + NT - 1) / NT;
+    double2 st[NE], sy = make_double2(0.0, 0.0);
+    auto back_load = [&](int j1) {
+      const int j0 = max(1, j1 - kBcBack + 1);
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        const int x = tid + NT * e, k = x % kBcBack, o = b - x / kBcBack + k;
+        const int i = j0 + k - o;
+        st[e] = make_double2(0.0, 0.0);
+        if (o >= 0 && o <= b && j0 + k <= j1 && i >= 1) st[e] = U[(int64_t)(i - 1) * M + o];
       }
-      for (int e = tid; e < cnt; e += nt) {
-        const int jj = j0 + e;
-        double2 v = make_double2(0.0, 0.0);
-        if (jj - b >= 1) v = Y[jj - b - 1];
-        W[b * B1 + e] = v;
-      }
+      sy = make_double2(0.0, 0.0);
+      if (tid < kBcBack && j0 + tid - 128 >= 1) sy = Y[j0 + tid - 128 - 1];
+    };
+    double2 ya = make_double2(0.0, 0.0), yb = ya;
+    if (wave == 0) {
+      const int ra = n - ((n - lane) & 63);
+      if (ra >= 1) ya = Y[ra - 1];
+      if (ra > 64) yb = Y[ra - 65];
+    }
+    // (arrived here: pending at the steps, they would make each step wait for
+    // the next chunk's loads too)
+    asm volatile("" : "+v"(ya.x), "+v"(ya.y), "+v"(yb.x), "+v"(yb.y));
+    back_load(n);
+    for (int j1 = n; j1 >= 1; j1 -= kBcBack) {
+      const int j0 = max(1, j1 - kBcBack + 1);
       __syncthreads();
-      if (tid < 64) {
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        const int x = tid + NT * e, k = x % kBcBack, o = b - x / kBcBack + k;
+        if (o >= 0 && o <= b) SU[k * B1 + o] = st[e];
+      }
+      if (tid < kBcBack) SY[tid] = sy;
+      __syncthreads();
+      if (wave == 0 && lane < kBcBack) SD[lane] = bz_den(SU[lane * B1]);
+      sw_order();
+      if (j1 - kBcBack >= 1) back_load(j1 - kBcBack);
+      if (wave == 0) {
+        // a step's reads a step ahead; column entry o past the band or above
+        // row 1 is taken as 0 (subtracting x*0 changes nothing)
+        double2 ua, ub, ys;
+        BzDen p;
+        auto fetch = [&](int j) {
+          const int k = j - j0, o = (j - lane) & 63;
+          const double2* Uc = SU + k * B1;
+          p = SD[k];
+          ys = SY[k];
+          const double2 va = Uc[min(o, b)], vb = Uc[min(o + 64, b)];
+          const bool oa = o >= 1 && o <= b, ob = o + 64 <= b;
+          ua = make_double2(oa ? va.x : 0.0, oa ? va.y : 0.0);
+          ub = make_double2(ob ? vb.x : 0.0, ob ? vb.y : 0.0);
+        };
+        fetch(j1);
         for (int j = j1; j >= j0; --j) {
-          const double2* Uc = W + (j - j0) * B1;
-          const double2 yj = Bv[j % B1];
-          const bool go = bz_nz(yj);
+          const BzDen pj = p;
+          const double2 uaj = ua, ubj = ub, ysj = ys;
+          fetch(max(j - 1, j0));
+          const int lj = j & 63;
+          const double2 yj = bc_lane(ya, lj);
           double2 xj = yj;
-          if (go) xj = bz_div(yj, Uc[0]);
-          const int om = min(b, j - 1);
-          for (int o = 1 + tid; o <= om; o += 64) {
-            const int sr = (j - o) % B1;
-            double2 v;
-            if (o == b) v = W[b * B1 + (j - j0)];
-            else v = Bv[sr];
-            if (go) {
-              const double2 u = bz_mul(xj, Uc[o]);
-              v = make_double2(v.x - u.x, v.y - u.y);
-            }
-            Bv[sr] = v;
+          if (bz_nz(yj)) {   // uniform
+            xj = bz_div(yj, pj);
+            const double2 da = bz_mul(xj, uaj), db = bz_mul(xj, ubj);
+            ya = make_double2(ya.x - da.x, ya.y - da.y);
+            yb = make_double2(yb.x - db.x, yb.y - db.y);
           }
-          if (tid == 0) Y[j - 1] = xj;
-          wave_sync();
+          if (lane == lj) {
+            SX[j - j0] = xj;
+            ya = yb;
+            yb = ysj;
+          }
         }
+        if (lane <= j1 - j0) Y[j0 + lane - 1] = SX[lane];
       }
     }
     __syncthreads();
     // Esol into the edge field (mode 2: x-edges of x-slice s; mode 1: y-edges
     // of y-slice s); the bottom face carries the zeroed xZMax / yZMax
-    const int nzp = a.nz + 1, nhp = Ny + 1;
+    const BcArgs a = *bc_reload(ap);
+    const BcSlice S = bc_slice(a, it);
+    const double2* exb = a.exb + (int64_t)it * a.mmbMax;
+    const int Ny = S.nh, nzp = a.nz + 1, nhp = Ny + 1;
     double2* E = a.e + (int64_t)S.sys * a.nE;
-    for (int e = tid; e < nhp * nzp; e += nt) {
+    for (int e = tid; e < nhp * nzp; e += NT) {
       const int iz = 1 + e % nzp, ih = 1 + e / nzp;
       double2 v;
       if (iz == nzp) v = make_double2(0.0, 0.0);

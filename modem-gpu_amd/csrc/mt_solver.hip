@@ -1423,6 +1423,22 @@ static int download_padded(mt_ctx* ctx, int nsys, const Z* d, mt_zdouble* h, con
   return MT_OK;
 }
 
+// The slice kernel for nz: the smallest register window that holds it (the
+// entry point takes nz to about 100).
+struct BcKernel { const void* f; int threads, slots; };
+template <int TG, int R>
+static BcKernel bc_shape() {
+  return {reinterpret_cast<const void*>(&k_bc_te2d<TG, R>), TG * TG, TG * R};
+}
+static BcKernel bc_kernel(int nz) {
+  if (nz <= 32) return bc_shape<16, 2>();
+  if (nz <= 48) return bc_shape<16, 3>();
+  if (nz <= 64) return bc_shape<16, 4>();
+  if (nz <= 80) return bc_shape<16, 5>();
+  if (nz <= 96) return bc_shape<16, 6>();
+  return bc_shape<16, 7>();
+}
+
 extern "C" {
 
 void mt_default_opts(mt_solve_opts* o) {
@@ -1931,11 +1947,11 @@ int mt_bc_x0_dev(mt_ctx* ctx, int nsys, const double* omegas, const int* modes, 
     if ((modes[s] != 1 && modes[s] != 2) || !(omegas[s] > 0.0))
       return mt_fail(ctx, MT_E_ARG, "mt_bc_x0_dev: mode must be 1 or 2 and omega > 0");
   MT_HIP_CHECK(ctx, hipSetDevice(ctx->device));
-  const size_t lds = bc_lds_bytes(nz);
   int maxlds = 0;
   MT_HIP_CHECK(ctx, hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device));
-  if (lds + 64 > size_t(maxlds))
-    return mt_fail(ctx, MT_E_ARG, "mt_bc_x0_dev: nz too large for the slice window in LDS");
+  if (bc_window_bytes(nz) + 64 > size_t(maxlds) || nz > 112)
+    return mt_fail(ctx, MT_E_ARG, "mt_bc_x0_dev: nz too large for the slice window");
+  const BcKernel bk = bc_kernel(nz);
   // host side: earth conductivities as ModelParamToCell forms them, block distances, items
   const int64_t nce = int64_t(nx) * ny * H.nzEarth;
   std::vector<double> sig(nce);
@@ -1957,20 +1973,24 @@ int mt_bc_x0_dev(mt_ctx* ctx, int nsys, const double* omegas, const int* modes, 
   const int nitem = int(items.size());
   const int nhmax = std::max(nx, ny), b = nz - 1;
   const int64_t nmax = int64_t(nhmax - 1) * b;
-  const int per_cu = 2 * (lds + 64) <= size_t(160 * 1024) ? 2 : 1;   // workgroups per CU by LDS (160 KB)
-  const int G = std::max(1, std::min(nitem, ctx->num_cu * per_cu));
+  // one slice per workgroup; as many workgroups as are resident at once, fewer
+  // where their scratch does not fit
+  const size_t lds = bc_back_bytes(nz);
+  int per_cu = 0;
+  MT_HIP_CHECK(ctx, hipFuncSetAttribute(bk.f, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+  MT_HIP_CHECK(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, bk.f, bk.threads, lds));
+  int G = std::max(1, std::min(nitem, ctx->num_cu * std::max(1, per_cu)));
   BcArgs a;
   a.nx = nx; a.ny = ny; a.nz = nz; a.nza = nza;
   a.nXe = g.nXe; a.nE = g.nE;
   a.nitem = nitem;
   a.ncolMax = nhmax + 1;
   a.mmbMax = 2 * nhmax + 2 * nz + 1;
-  a.uStride = nmax * nz;
-  a.yStride = nmax;
   double *ddx, *ddy, *ddz, *dcx, *dcy, *dcz, *dsig, *dom;
   int *dmode, *dflag;
   int2* ditem;
-  double2 *dexb, *dside, *du, *dy;
+  double2 *dexb, *dside, *du = nullptr, *dy = nullptr;
+  BcCoef* dcoef = nullptr;
   int rc;
   if ((rc = ws(ctx, "bc_dx", nx, &ddx)) || (rc = ws(ctx, "bc_dy", ny, &ddy)) ||
       (rc = ws(ctx, "bc_dz", nz, &ddz)) || (rc = ws(ctx, "bc_cx", nx + 1, &dcx)) ||
@@ -1979,10 +1999,15 @@ int mt_bc_x0_dev(mt_ctx* ctx, int nsys, const double* omegas, const int* modes, 
       (rc = ws(ctx, "bc_mode", nsys, &dmode)) || (rc = ws(ctx, "bc_item", nitem, &ditem)) ||
       (rc = ws(ctx, "bc_flag", nitem, &dflag)) ||
       (rc = ws(ctx, "bc_exb", size_t(nitem) * a.mmbMax, &dexb)) ||
-      (rc = ws(ctx, "bc_side", size_t(nitem) * 4 * nz, &dside)) ||
-      (rc = ws(ctx, "bc_u", size_t(G) * a.uStride, &du)) ||
-      (rc = ws(ctx, "bc_y", size_t(G) * a.yStride, &dy)))
+      (rc = ws(ctx, "bc_side", size_t(nitem) * 4 * nz, &dside)))
     return rc;
+  for (;; G = (G + 1) / 2) {
+    if (!(rc = ws(ctx, "bc_u", size_t(G) * nmax * bk.slots, &du)) &&
+        !(rc = ws(ctx, "bc_y", size_t(G) * nmax, &dy)) &&
+        !(rc = ws(ctx, "bc_coef", size_t(G) * nmax, &dcoef)))
+      break;
+    if (rc != MT_E_OOM || G == 1) return rc;
+  }
   MT_HIP_CHECK(ctx, hipMemcpy(ddx, H.dx.data(), nx * sizeof(double), hipMemcpyHostToDevice));
   MT_HIP_CHECK(ctx, hipMemcpy(ddy, H.dy.data(), ny * sizeof(double), hipMemcpyHostToDevice));
   MT_HIP_CHECK(ctx, hipMemcpy(ddz, H.dz.data(), nz * sizeof(double), hipMemcpyHostToDevice));
@@ -1995,15 +2020,19 @@ int mt_bc_x0_dev(mt_ctx* ctx, int nsys, const double* omegas, const int* modes, 
   MT_HIP_CHECK(ctx, hipMemcpy(ditem, items.data(), nitem * sizeof(int2), hipMemcpyHostToDevice));
   a.dx = ddx; a.dy = ddy; a.dz = ddz; a.cx = dcx; a.cy = dcy; a.cz = dcz;
   a.sig = dsig; a.omega = dom; a.mode = dmode; a.item = ditem;
-  a.exb = dexb; a.side = dside; a.ucol = du; a.yx = dy; a.flag = dflag;
+  a.exb = dexb; a.side = dside; a.flag = dflag;
   a.e = static_cast<double2*>(e_dev);
   MT_HIP_CHECK(ctx, hipMemsetAsync(e_dev, 0, size_t(nsys) * g.nE * sizeof(double2), ctx->stream));
   const int64_t n1 = int64_t(nitem) * a.ncolMax;
   k_bc_te1d<<<unsigned((n1 + 255) / 256), 256, 0, ctx->stream>>>(a);
   MT_HIP_CHECK(ctx, hipGetLastError());
-  MT_HIP_CHECK(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_bc_te2d),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-  k_bc_te2d<<<unsigned(G), 256, lds, ctx->stream>>>(a);
+  BcArgs* da;
+  if ((rc = ws(ctx, "bc_args", 1, &da))) return rc;
+  MT_HIP_CHECK(ctx, hipMemcpyAsync(da, &a, sizeof(a), hipMemcpyHostToDevice, ctx->stream));
+  const BcArgs* dap = da;
+  BcScratch scr = {du, dy, dcoef, nmax, nz, nitem};
+  void* kargs[] = {&dap, &scr};
+  MT_HIP_CHECK(ctx, hipLaunchKernel(bk.f, dim3(unsigned(G)), dim3(unsigned(bk.threads)), kargs, lds, ctx->stream));
   MT_HIP_CHECK(ctx, hipGetLastError());
   std::vector<int> flags(nitem);
   MT_HIP_CHECK(ctx, hipMemcpyAsync(flags.data(), dflag, nitem * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));

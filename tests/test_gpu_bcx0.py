@@ -150,3 +150,24 @@ def test_bc_x0_dev_argument_errors(gpu_ctx):
         with pytest.raises(mtsp2.MTError) as ei:
             ctx.bc_x0(np.array(om), np.array(md))
         assert ei.value.code == mtsp2.MT_E_ARG
+
+
+@pytest.mark.parametrize("nz", [3, 32, 33, 48, 49, 64, 65, 80, 81, 96, 97, 100])
+def test_bc_x0_dev_window_edges(gpu_ctx, nz):
+    """The register windows of the slice solver at the ends of their ranges of
+    nz, slices of one to five node columns, and frequencies from a static
+    field to one that decays into the denormal range (the quotients' plain
+    division): bit for bit against the oracle."""
+    print(f"case bc_x0 window nz={nz}", flush=True)
+    nza = max(1, nz // 5)
+    rng = np.random.default_rng(nz)
+    for nx, ny in ((2, 6), (5, 3)):
+        dx, dy = rng.uniform(100, 300, nx), rng.uniform(100, 300, ny)
+        dz = np.concatenate([np.geomspace(3e4, 100, nza), rng.uniform(50, 200, nz - nza)])
+        lc = -np.log(rng.uniform(1.0, 1000.0, (nx, ny, nz - nza)))
+        gpu_ctx.assemble(dx, dy, dz, nza, lc)
+        om = 2 * np.pi * np.array([1e-4, 3.0, 1e9])
+        for mode in (1, 2):
+            md = np.full(len(om), mode)
+            e = gpu_ctx.bc_x0(om, md)
+            assert np.array_equal(e, _want(dx, dy, dz, nza, lc, om, md)), (nx, ny, mode)
