@@ -22,6 +22,7 @@
 #pragma once
 
 #include "mt_kernels.hpp"
+#include "mt_sweep.hpp"
 
 namespace mt {
 
@@ -129,47 +130,28 @@ __device__ __forceinline__ int64_t lat_e(const LatticeInfo& L, int i, int j, int
 
 // ------------------------------------------ reference ordering, 8x8x8 tiles
 // One tile level per launch (grid = tiles of the level x active systems), one
-// wave per (tile, system): the tile's inputs and the upstream neighbours'
-// facing layer (final after the previous launch) are staged into LDS, the 22
-// hyperplanes swept, the tile written back.  A launch holds a few dozen to a
-// few hundred tiles of one system, so a tile's time is the launch's time, and
-// it is latency: the chain of dependent loads before the data arrive, the
-// hyperplane steps, the stores.
-//  * Loads: the system-independent tables (tile, lane's point of every
-//    hyperplane, level slots) and the system lookups are requested together,
-//    then every data load at once; the system's status is checked after (a
-//    skipped system's loads are wasted, never out of bounds).
-//  * A hyperplane step is one round of LDS reads: the lane's points are in
-//    registers (box index and level slot, extent folded in), the pivots and
-//    couplings sit by level slot (consecutive lanes, consecutive entries), and
-//    the box is rb_box's pitch-82 layout, which spreads a hyperplane over the
-//    LDS banks.
-//   forward: the box holds r on the tile and w = dinv*y of the low faces;
-//            a step forms y = r - sum a w, keeps y in the pivot's slot and
-//            leaves w = dinv*y in the box; y is written back.
-//   backward: the box holds y on the tile and z of the high faces (past the
-//             box's last plane, kRbNB + kRbPK entries in all); a step forms
-//             z = dinv*(y - sum a z) in place; z is written back.
-// Per point the three terms are taken in the order i, j, k.
+// wave per (tile, system): the tile is swept in registers (mt_sweep.hpp), the
+// upstream neighbours' facing layer (final after the previous launch) folded
+// into its right-hand side first.  A launch holds a few dozen to a few hundred
+// tiles of one system, so a tile's time is the launch's time, and it is
+// latency: the chain of dependent loads before the data arrive, the sweep, the
+// stores.  Every data load is issued before the system's status is checked (a
+// skipped system's loads are wasted, never out of bounds).
+//   forward: y = r - sum a w kept, w = dinv*y passed on; y is written back.
+//   backward: in place on y, z = dinv*(y - sum a z); z is written back.
+// Measured at FP64, one system, per application (two sweeps): 100x100x60+10, 66
+// levels, 565 us swept out of an LDS box, 449 in registers (6.8 us a level, of
+// which the sweep is about 1); 40x40x30+10 205 and 157.
 template <class T, class V, bool FWD>
-__global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a, const TileShape* __restrict__ shp) {
-  constexpr int TX = 8, NP = kRbNP, NU = 8, NLEV = 22;
-  constexpr int NB = FWD ? kRbNB : kRbNB + kRbPK;
-  struct Cpl { V c[3]; };
-  __shared__ C2<T> W[NB];
-  __shared__ C2<T> DV[NP];   // pivots by level slot (forward: then y)
-  __shared__ Cpl CF[NP];     // the sweep's couplings by level slot
+__global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a) {
+  constexpr int TX = 8, NP = kRbNP, NU = 8;
+  __shared__ C2<T> P[NP];     // the tile, point order
+  __shared__ V CF[3][NP];     // the sweep's couplings
+  __shared__ C2<T> X[64];     // cross-row words of the sweep
   const int lane = threadIdx.x;
   const int tix = blockIdx.x / a.nact, si = blockIdx.x - tix * a.nact;
-  // ---- system-independent tables and the system lookups, together
   const int4 tl = a.tiles[tix];
   const int sys = a.act[si];
-  int sl[NU];
-#pragma unroll
-  for (int u = 0; u < NU; ++u) sl[u] = shp->rslot[lane + 64 * u];
-  unsigned int pv[NLEV];
-#pragma unroll
-  for (int h = 0; h < NLEV; ++h) pv[h] = shp->lpts[h][lane];
   const SysScal& sc = a.sc[sys];
   const int status = sc.status, fidx = sc.fidx;
   const LatticeInfo L = a.lat[tl.x];
@@ -180,7 +162,6 @@ __global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a, const TileShap
   const C2<T>* __restrict__ pout = a.out + o;
   const C2<T>* __restrict__ dinv = a.dinv + (int64_t)fidx * cst;
   const V* __restrict__ cf0 = a.coef + (FWD ? 1 : 2) * cst;   // slots 1,3,5 / 2,4,6
-  const int st[3] = {1, kRbBX, kRbPK};
   // ---- the tile's own data (p = lane + 64u: li = lane&7, lj = lane>>3,
   // lk = u): forward r (- alpha*in2), backward y; pivots; couplings
   const int li0 = lane & 7, lj0 = lane >> 3;
@@ -207,9 +188,10 @@ __global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a, const TileShap
     }
   }
   // the facing layer of the upstream neighbours (forward: low faces, y and
-  // pivot; backward: high faces, z)
+  // pivot; backward: high faces, z), with the coupling across the face
   int fq[3];
   C2<T> fv[3], fd[3];
+  V fc[3];
 #pragma unroll
   for (int dir = 0; dir < 3; ++dir) {
     const int t0 = FWD ? 0 : TX - 1;
@@ -221,95 +203,82 @@ __global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a, const TileShap
     const int nj = gj0 + tj + (dir == 1 ? d : 0);
     const int nk = gk0 + tk + (dir == 2 ? d : 0);
     fv[dir] = fd[dir] = {T(0), T(0)};
-    fq[dir] = -1;
+    fc[dir] = V(0);
+    fq[dir] = ti + TX * (tj + TX * tk);
     const bool ok = ti < ex && tj < ey && tk < ez && ni >= 0 && nj >= 0 && nk >= 0 &&
                     ni < L.A && nj < L.B && nk < L.C;
     if (ok) {
       const int64_t l = lat_e(L, ni, nj, nk);
       fv[dir] = pout[l];
       if (FWD) fd[dir] = dinv[l];
-      fq[dir] = FWD ? rb_box(ti, tj, tk) - st[dir] : rb_box(ti, tj, tk) + st[dir];
+      fc[dir] = cf0[(int64_t)(2 * dir) * cst + lat_e(L, gi0 + ti, gj0 + tj, gk0 + tk)];
     }
   }
   if (status != a.status_req) return;   // uniform
-  // this lane's point on every hyperplane: box index | level slot << 10
-  unsigned int pk[NLEV];
+  const int skew = sw_skew(lane);
+  // ---- pivots, couplings (0 across the tile's faces) and the right-hand side
+  // into skewed registers
 #pragma unroll
-  for (int h = 0; h < NLEV; ++h) {
-    const unsigned int v = pv[h];
-    const int li = v & 7, lj = (v >> 3) & 7, lk = (v >> 6) & 7;
-    const bool ok = v != 0xffffffffu && li < ex && lj < ey && lk < ez;
-    pk[h] = ok ? (unsigned(rb_box(li, lj, lk)) | ((v >> 9) << 10)) : 0xffffffffu;
+  for (int u = 0; u < NU; ++u) {
+    const int p = lane + 64 * u, t0 = FWD ? 0 : TX - 1;
+    P[p] = dd[u];
+    CF[0][p] = li0 == t0 ? V(0) : cc[u][0];
+    CF[1][p] = lj0 == t0 ? V(0) : cc[u][1];
+    CF[2][p] = u == t0 ? V(0) : cc[u][2];
   }
-  // ---- stage: zero box (partial tiles and absent faces read zeros), then
-  // the tile, the faces, the per-slot data
-  for (int q = lane; q < NB; q += 64) W[q] = {T(0), T(0)};
+  X[lane] = {T(0), T(0)};
+  wave_sync();
+  C2<T> D[NU], R[NU];
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int p = sw_point(lane, skew, u);
+    D[u] = P[p];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) cc[u][s] = CF[s][p];
+  }
   wave_sync();
   const C2<T> al = ccast<T>(sc.alpha);
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
     C2<T> r = rv[u];
     if (FWD && a.in2) r = csub(r, cmul(al, r2[u]));
-    W[rb_box(li0, lj0, u)] = r;
-    DV[sl[u]] = dd[u];
-    Cpl c;
-#pragma unroll
-    for (int s = 0; s < 3; ++s) c.c[s] = cc[u][s];
-    CF[sl[u]] = c;
+    P[lane + 64 * u] = r;
   }
-#pragma unroll
-  for (int dir = 0; dir < 3; ++dir)
-    if (fq[dir] >= 0) W[fq[dir]] = FWD ? cmul(fd[dir], fv[dir]) : fv[dir];
   wave_sync();
-  if (FWD) {
 #pragma unroll
-    for (int h = 0; h < NLEV; ++h) {
-      const unsigned int pt = pk[h];
-      if (pt != 0xffffffffu) {
-        const int q = pt & 0x3ff, p = pt >> 10;
-        const C2<T> dvp = DV[p];
-        const Cpl c = CF[p];
-        C2<T> y = W[q];
-#pragma unroll
-        for (int s = 0; s < 3; ++s) {
-          const T cs = T(c.c[s]);
-          const C2<T> w = W[q - st[s]];
-          y.x -= cs * w.x;
-          y.y -= cs * w.y;
-        }
-        DV[p] = y;
-        W[q] = cmul(dvp, y);
-      }
-      wave_sync();
-    }
-  } else {
-#pragma unroll
-    for (int h = NLEV - 1; h >= 0; --h) {
-      const unsigned int pt = pk[h];
-      if (pt != 0xffffffffu) {
-        const int q = pt & 0x3ff, p = pt >> 10;
-        const C2<T> dvp = DV[p];
-        const Cpl c = CF[p];
-        C2<T> y = W[q];
-#pragma unroll
-        for (int s = 0; s < 3; ++s) {
-          const T cs = T(c.c[s]);
-          const C2<T> z = W[q + st[s]];
-          y.x -= cs * z.x;
-          y.y -= cs * z.y;
-        }
-        W[q] = cmul(dvp, y);
-      }
-      wave_sync();
-    }
+  for (int dir = 0; dir < 3; ++dir) {   // one direction after another: a tile edge lies on two faces
+    const C2<T> w = FWD ? cmul(fd[dir], fv[dir]) : fv[dir];
+    const T c = T(fc[dir]);
+    C2<T> r = P[fq[dir]];
+    r.x -= c * w.x;
+    r.y -= c * w.y;
+    P[fq[dir]] = r;
+    wave_sync();
   }
+#pragma unroll
+  for (int u = 0; u < NU; ++u) R[u] = P[sw_point(lane, skew, u)];
+  sw_run<!FWD>(lane, skew, X, [&](int u, C2<T> vi, C2<T> vj, C2<T> vk, bool act) {
+    C2<T> y = R[u];
+    y.x -= T(cc[u][0]) * vi.x;
+    y.y -= T(cc[u][0]) * vi.y;
+    y.x -= T(cc[u][1]) * vj.x;
+    y.y -= T(cc[u][1]) * vj.y;
+    y.x -= T(cc[u][2]) * vk.x;
+    y.y -= T(cc[u][2]) * vk.y;
+    const C2<T> z = cmul(D[u], y);
+    const C2<T> keep = FWD ? y : z;
+    R[u] = {act ? keep.x : R[u].x, act ? keep.y : R[u].y};
+    return z;
+  });
   // ---- write the tile back: forward y, backward z
+  wave_sync();
+#pragma unroll
+  for (int u = 0; u < NU; ++u) P[sw_point(lane, skew, u)] = R[u];
+  wave_sync();
   C2<T>* __restrict__ dst = a.out + o;
 #pragma unroll
-  for (int u = 0; u < NU; ++u) {
-    if (!(col_ok && u < ez)) continue;
-    dst[e0 + u * kst] = FWD ? DV[sl[u]] : W[rb_box(li0, lj0, u)];
-  }
+  for (int u = 0; u < NU; ++u)
+    if (col_ok && u < ez) dst[e0 + u * kst] = P[lane + 64 * u];
 }
 
 // ------------------------------------------------- red-black tile ordering

@@ -599,7 +599,7 @@ static void dilu_fwd(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
   for (int L = 0; L < tp.nlev; ++L) {
     a.tiles = tp.tiles + tp.lvl_off[L];
     a.ntiles = tp.lvl_off[L + 1] - tp.lvl_off[L];
-    k_dilu_ro<T, V, true><<<a.ntiles * a.nact, 64, 0, ctx->stream>>>(a, tp.shape);
+    k_dilu_ro<T, V, true><<<a.ntiles * a.nact, 64, 0, ctx->stream>>>(a);
   }
 }
 
@@ -609,7 +609,7 @@ static void dilu_bwd(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
   for (int L = tp.nlev - 1; L >= 0; --L) {
     a.tiles = tp.tiles + tp.lvl_off[L];
     a.ntiles = tp.lvl_off[L + 1] - tp.lvl_off[L];
-    k_dilu_ro<T, V, false><<<a.ntiles * a.nact, 64, 0, ctx->stream>>>(a, tp.shape);
+    k_dilu_ro<T, V, false><<<a.ntiles * a.nact, 64, 0, ctx->stream>>>(a);
   }
 }
 
