@@ -178,7 +178,7 @@ def main():
     ap.add_argument("--dilu-variant", type=int, default=6, choices=(1, 4, 5, 6),
                     help="red-black DILU launch shape: 1 single-system persistent, 4 four systems "
                          "per workgroup, 5 the same with the lean LDS layout, 6 as 5 with, for "
-                         "inner solves on bricks, the p-update folded into the red forward launch")
+                         "inner solves on bricks, the p-update folded into the forward launches")
     ap.add_argument("--drop-in-only", type=int, default=0, metavar="NSYS",
                     help="only the plain FP64 solves (one system at a time, reference-ordered "
                          "DILU: the cuBiCG drop-in) of the first NSYS forward systems, for profiling")

@@ -392,7 +392,7 @@ int mt_set_spmv_variant(mt_ctx *ctx, int variant, int layers_per_segment);
  * couplings in LDS; 5 = the same with the lean LDS layout (three workgroups
  * per CU); 6 (default) = as 5, and in the inner solves on bricks, whose
  * sweeps are the same register sweeps for every variant, the p-update folded
- * into the red forward launch (variants 1 to 5 run it apart).  The same
+ * into the forward launches (variants 1 to 5 run it apart).  The same
  * operator; 5 and 6 round the black tiles' backward sweep differently from 1
  * and 4 (6 is bitwise 5).  No counterpart in the reference. */
 int mt_set_dilu_variant(mt_ctx *ctx, int variant);

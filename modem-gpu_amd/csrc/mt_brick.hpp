@@ -201,42 +201,6 @@ __global__ __launch_bounds__(BS) void k_bk_widen(const C2<float>* __restrict__ x
     y[q] = {double(x[q].x), double(x[q].y)};
 }
 
-// k_pupdate on the tiles of one colour of the red-black plan (tiles[0,
-// ntiles): {lattice, ti, tj, tk}): the black tiles' p, when the red forward
-// sweep forms the red tiles' itself.  Block (system, chunk g of the tiles),
-// as k_pupdate's; the same arithmetic per point.
-template <class T, class V>
-__global__ __launch_bounds__(BS) void k_pupdate_tiles(IterArgs<T, V> a, const int4* __restrict__ tiles,
-                                                      int ntiles, LatticeInfo l0, LatticeInfo l1,
-                                                      LatticeInfo l2) {
-  int si, g;
-  map_sys_block(a.nact, a.G, si, g);
-  const int sys = a.act[si];
-  const SysScal& sc = a.sc[sys];
-  if (sc.status != ST_RUN) return;
-  const int64_t o = (int64_t)sys * a.nE;
-  const bool rs = sc.restart_due;
-  const C2<T> beta = ccast<T>(sc.beta), om = ccast<T>(sc.omg);
-  const int t0 = int(int64_t(ntiles) * g / a.G), t1 = int(int64_t(ntiles) * (g + 1) / a.G);
-  for (int t = t0; t < t1; ++t) {
-    const int4 tl = tiles[t];
-    const LatticeInfo L = tl.x == 0 ? l0 : (tl.x == 1 ? l1 : l2);
-    const int64_t b0 = o + (int64_t)(L.tbase + tl.y + L.ntx * (tl.z + L.nty * tl.w)) * kBkPts;
-    for (int q = threadIdx.x; q < kBkPts; q += BS) {
-      const int64_t e = b0 + q;
-      const C2<T> r = a.r[e];
-      C2<T> p;
-      if (rs) {
-        a.rt[e] = r;
-        p = r;
-      } else {
-        p = cadd(r, cmul(beta, csub(a.p[e], cmul(om, a.v[e]))));
-      }
-      a.p[e] = p;
-    }
-  }
-}
-
 // Point p of tile t for the brick SpMV: whether it is an interior edge, its
 // brick index e, its 14 neighbours' brick indices (a neighbour that is not an
 // interior edge has a zero coupling and the row's own index) and its 16
@@ -537,8 +501,8 @@ __global__ __launch_bounds__(kBtThreads, 4) void k_spmv_btp(IterArgs<float, floa
 // tiles contribute (black: all six faces before the forward sweep; red: all
 // six before the backward one, the forward one has none) is folded into the
 // right-hand side first, so the sweeps' couplings out of the tile are zero.
-// PU: the red forward sweep of the first application forms the BiCGStab
-// p = r + beta (p - omega v) for its tiles as it loads them.
+// PU: the forward sweeps of the first application form the BiCGStab
+// p = r + beta (p - omega v) for their tiles as they load them.
 // DiluArgs on bricks: coef = the [6][nB] couplings (slots 1..6), cstride =
 // nB, vstride = nB, dinv = [nfreq][nB].
 // What bounds it: memory at many systems (100x100x60+10, 16 systems: red
@@ -552,7 +516,7 @@ __global__ __launch_bounds__(kBtThreads, 4) void k_spmv_btp(IterArgs<float, floa
 template <class T, class V, int MODE, int NW, bool ZP = false, bool PU = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? (PU ? 4 : 5) : 1) void k_dilu_bc(DiluArgs<T, V> a) {
   constexpr int TX = 8, NP = kRbNP, NU = 8;
-  static_assert(!PU || MODE == RB_RED_FWD, "the p-update is folded into the red forward sweep");
+  static_assert(!PU || MODE != RB_RED_BWD, "the p-update is folded into the forward sweeps");
   constexpr bool FWDP = MODE != RB_RED_BWD;   // has a forward sweep
   constexpr bool BWDP = MODE != RB_RED_FWD;   // has a backward sweep
   constexpr bool HALO = MODE != RB_RED_FWD;   // reads face neighbours
@@ -711,7 +675,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? (PU ? 4 : 5) : 1) void k_dilu_bc
     C2<T> r = rv[u];
     const int64_t pe = o + tb + lane + 64 * u;
     if constexpr (PU) {
-      // k_pupdate's p, stored for the red tiles
+      // k_pupdate's p, stored for the colour's tiles
       if (sc.restart_due) {
         a.pu_rt[pe] = r3[u];
         r = r3[u];

@@ -102,11 +102,10 @@ struct DiluArgs {
   // the black tiles' j- and k-faces from zout
   C2<T>* zout = nullptr;
   int64_t zpair = 0;
-  // red forward sweep of the first application on bricks, when pu_r is set:
-  // its right-hand side is the BiCGStab p = r + beta (p - omega v) (on a
-  // restart p = r and rt = r), formed from r (pu_r), the previous p (in) and
-  // v (pu_v), and stored (pu_p, pu_rt) for the red tiles (the black tiles'
-  // by k_pupdate_tiles before the launch)
+  // forward sweeps of the first application on bricks, when pu_r is set: their
+  // right-hand side is the BiCGStab p = r + beta (p - omega v) (on a restart
+  // p = r and rt = r), formed from r (pu_r), the previous p (in) and v (pu_v),
+  // and stored (pu_p, pu_rt)
   const C2<T>* pu_r = nullptr;
   const C2<T>* pu_v = nullptr;
   C2<T>* pu_p = nullptr;

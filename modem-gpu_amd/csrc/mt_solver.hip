@@ -160,7 +160,7 @@ struct mt_ctx {
                                 // 5 the same in the lean LDS layout; 6 as 5,
                                 // and on bricks (where every variant runs
                                 // k_dilu_bc) the p-update folded into the
-                                // red forward launch
+                                // forward launches
   // kernel timing (mt_timing_enable): HIP events on `stream` around every
   // SpMV launch and every DILU sweep of the BiCGStab engine
   bool timing = false;
@@ -680,8 +680,10 @@ static void dilu_bk_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<float, float
       constexpr int NW = decltype(nwc)::value;
       constexpr bool ZP = decltype(zp)::value;
       const hipStream_t st = ctx->stream;
-      if (step == 0 && a.pu_r)   // (the p-update folded into the red forward sweep)
+      if (step == 0 && a.pu_r)   // (the p-update folded into the forward sweeps)
         k_dilu_bc<float, float, RB_RED_FWD, NW, ZP, true><<<g, 64 * NW, 0, st>>>(a);
+      else if (step == 1 && a.pu_r)
+        k_dilu_bc<float, float, RB_BLACK_FB, NW, ZP, true><<<g, 64 * NW, 0, st>>>(a);
       else if (step == 0) k_dilu_bc<float, float, RB_RED_FWD, NW, ZP><<<g, 64 * NW, 0, st>>>(a);
       else if (step == 1) k_dilu_bc<float, float, RB_BLACK_FB, NW, ZP><<<g, 64 * NW, 0, st>>>(a);
       else k_dilu_bc<float, float, RB_RED_BWD, NW, ZP><<<g, 64 * NW, 0, st>>>(a);
@@ -831,7 +833,7 @@ struct Engine {
   // out = M^-1 (in - alpha*in2) (in2 may be null); with zout (bricks, paired
   // x) the result goes to zout pair-interleaved and out holds the red tiles'
   // intermediate w
-  // pu: the red forward sweep also forms p (k_pupdate) for the red tiles
+  // pu: the forward sweeps also form p (k_pupdate)
   void precond(const C2<T>* in, C2<T>* out, const C2<T>* in2 = nullptr, C2<T>* zout = nullptr,
                bool pu = false) {
     if (a.pc != PCK_DILU && a.pc != PCK_DILU_RB) return;
@@ -900,8 +902,8 @@ struct Engine {
     return G;
   }
 
-  // the p-update folded into the first application's red forward sweep:
-  // inner solves on bricks
+  // the p-update folded into the first application's forward sweeps: inner
+  // solves on bricks
   bool pfold() const {
     return brick && a.fused && a.pc == PCK_DILU_RB && ctx->rb_variant == 6 && ctx->tiles_rb.nlev == 2;
   }
@@ -910,10 +912,7 @@ struct Engine {
     hipStream_t s = ctx->stream;
     // (paired x: p-hat to phi, the sweeps' w in ph)
     if (pfold()) {
-      // p of the black tiles here, of the red ones in the red forward sweep
-      const TilePlan& tp = ctx->tiles_rb;
-      k_pupdate_tiles<T, V><<<nblk, BS, 0, s>>>(a, tp.tiles + tp.lvl_off[1], tp.lvl_off[2] - tp.lvl_off[1],
-                                                tp.lat[0], tp.lat[1], tp.lat[2]);
+      // p formed by the forward sweeps as they load their tiles
       precond(a.p, a.ph, nullptr, a.ppair ? a.phi : nullptr, true);
     } else {
       k_pupdate<T, V><<<nblk, BS, 0, s>>>(a);
@@ -1017,11 +1016,10 @@ struct Engine {
                                    2.0 * units * 3.0 * n * sc2;
     // (the second application of an iteration reads r and v when fused, and
     // on bricks writes s = r - alpha v as well; with the p-update folded, the
-    // first one's red forward sweep reads r and v and writes p for the red
-    // tiles, half of the points)
+    // first one's forward sweeps read r and v too and write p)
     if (cnt[MT_KT_PRECOND])
       ctx->kt[MT_KT_PRECOND].bytes += cnt[MT_KT_PRECOND] * 6.0 * n * sv +
-                                      units * (3.0 + (pfold() ? 1.5 : 0.0) +
+                                      units * (3.0 + (pfold() ? 3.0 : 0.0) +
                                                (a.fused ? (a.s_ok ? 5.0 : 4.0) : 3.0)) * n * sc2;
     return MT_OK;
   }
