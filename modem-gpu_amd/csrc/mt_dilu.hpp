@@ -121,7 +121,47 @@ struct DiluArgs {
   // one coalesced read instead of 64 reads of 8 bytes, one per cache line.
   C2<T>* xf = nullptr;
   int64_t xfsys = 0, xfhalf = 0;
+  // the single-launch reference-ordered sweep (k_dilu_ro, DF): the faces in
+  // transit and the launch's counters (DfCtl)
+  unsigned long long* mail = nullptr;
+  int64_t dftiles = 0;     // tiles per active system in mail
+  int* dfctl = nullptr;
+  SysScal* scw = nullptr;
 };
+
+// ------------------------------------ faces in transit between running tiles
+// A tile hands its facing layer to its downstream neighbour through a mailbox
+// of its own: [active system][tile][direction][64 entries] complex, every
+// 8-byte word either a value or kDfEmpty, written and polled word by word with
+// relaxed agent-scope atomics (coherent across the XCDs; no fence, whose
+// write-back of an L2 costs microseconds).  The one reader empties it again.
+// kDfEmpty is a signalling NaN pattern that no arithmetic result has.
+constexpr unsigned long long kDfEmpty = 0xfff7a5a5fff7a5a5ull;
+constexpr int kDfWords = 3 * 64;          // complex entries per tile and active system
+constexpr int kDfSpin = 1 << 16;          // polls before a wait gives up (about 0.1 s)
+// (a cache line each: the counters are atomics of every workgroup)
+enum : int { DF_TICKET = 0, DF_DONE = 64, DF_FAILED = 128, DF_NCTL = 192 };
+
+__device__ __forceinline__ unsigned long long df_load(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void df_store(unsigned long long* p, unsigned long long v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void df_put(unsigned long long* p, C2<T> v) {
+  constexpr int W = sizeof(C2<T>) / 8;
+  unsigned long long w[W];
+  __builtin_memcpy(w, &v, sizeof(v));
+#pragma unroll
+  for (int q = 0; q < W; ++q) df_store(p + q, w[q]);
+}
+// all of the words of the mailboxes empty, the counters zero
+__global__ void k_df_clear(unsigned long long* mail, int64_t n, int* ctl) {
+  for (int64_t q = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; q < n; q += int64_t(gridDim.x) * blockDim.x)
+    mail[q] = kDfEmpty;
+  if (blockIdx.x == 0 && threadIdx.x < DF_NCTL) ctl[threadIdx.x] = 0;
+}
 
 __device__ __forceinline__ int64_t lat_e(const LatticeInfo& L, int i, int j, int k) {
   return L.base + (i + L.oi) + int64_t(L.a) * ((j + L.oj) + int64_t(L.b) * (k + L.ok));
@@ -141,14 +181,26 @@ __device__ __forceinline__ int64_t lat_e(const LatticeInfo& L, int i, int j, int
 // Measured at FP64, one system, per application (two sweeps): 100x100x60+10, 66
 // levels, 565 us swept out of an LDS box, 449 in registers (6.8 us a level, of
 // which the sweep is about 1); 40x40x30+10 205 and 157.
-template <class T, class V, bool FWD>
-__global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a) {
-  constexpr int TX = 8, NP = kRbNP, NU = 8;
-  __shared__ C2<T> P[NP];     // the tile, point order
-  __shared__ V CF[3][NP];     // the sweep's couplings
-  __shared__ C2<T> X[64];     // cross-row words of the sweep
-  const int lane = threadIdx.x;
-  const int tix = blockIdx.x / a.nact, si = blockIdx.x - tix * a.nact;
+template <class T, class V, bool FWD, bool DF>
+struct RoLds {
+  C2<T> P[kRbNP];   // the tile, point order
+  V CF[3][kRbNP];   // the sweep's couplings
+  C2<T> X[64];      // cross-row words of the sweep
+  C2<T> PD[FWD && DF ? kRbNP : 1];   // pivots, point order
+};
+
+// The sweep of item `work` (tile, active system) by one wave.
+template <class T, class V, bool FWD, bool DF>
+__device__ __forceinline__ void ro_tile(const DiluArgs<T, V>& a, RoLds<T, V, FWD, DF>& lds, int work) {
+  constexpr int TX = 8, NU = 8;
+  auto& P = lds.P;
+  auto& CF = lds.CF;
+  auto& X = lds.X;
+  auto& PD = lds.PD;
+  const int lane = threadIdx.x & 63;
+  int tix = work / a.nact;
+  const int si = work - tix * a.nact;
+  if (DF && !FWD) tix = a.ntiles - 1 - tix;   // (the tiles lie in level order)
   const int4 tl = a.tiles[tix];
   const int sys = a.act[si];
   const SysScal& sc = a.sc[sys];
@@ -189,6 +241,7 @@ __global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a) {
   // the facing layer of the upstream neighbours (forward: low faces, y and
   // pivot; backward: high faces, z), with the coupling across the face
   int fq[3];
+  bool fok[3];
   C2<T> fv[3], fd[3];
   V fc[3];
 #pragma unroll
@@ -206,10 +259,11 @@ __global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a) {
     fq[dir] = ti + TX * (tj + TX * tk);
     const bool ok = ti < ex && tj < ey && tk < ez && ni >= 0 && nj >= 0 && nk >= 0 &&
                     ni < L.A && nj < L.B && nk < L.C;
+    fok[dir] = ok;
     if (ok) {
       const int64_t l = lat_e(L, ni, nj, nk);
-      fv[dir] = pout[l];
-      if (FWD) fd[dir] = dinv[l];
+      if (!DF) fv[dir] = pout[l];
+      if (FWD && !DF) fd[dir] = dinv[l];
       fc[dir] = cf0[(int64_t)(2 * dir) * cst + lat_e(L, gi0 + ti, gj0 + tj, gk0 + tk)];
     }
   }
@@ -221,6 +275,7 @@ __global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a) {
   for (int u = 0; u < NU; ++u) {
     const int p = lane + 64 * u, t0 = FWD ? 0 : TX - 1;
     P[p] = dd[u];
+    if (FWD && DF) PD[p] = dd[u];
     CF[0][p] = li0 == t0 ? V(0) : cc[u][0];
     CF[1][p] = lj0 == t0 ? V(0) : cc[u][1];
     CF[2][p] = u == t0 ? V(0) : cc[u][2];
@@ -244,9 +299,46 @@ __global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a) {
     P[lane + 64 * u] = r;
   }
   wave_sync();
+  const int tself = L.tbase + tl.y + L.ntx * (tl.z + L.nty * tl.w);
+  constexpr int W = sizeof(C2<T>) / 8;
+  if constexpr (DF) {
+    unsigned long long* mb = a.mail + (int64_t(si) * a.dftiles + tself) * (kDfWords * W) + lane * W;
+    unsigned long long w[3][W];
+#pragma unroll
+    for (int dir = 0; dir < 3; ++dir)
+#pragma unroll
+      for (int q = 0; q < W; ++q) w[dir][q] = fok[dir] ? kDfEmpty : 0;
+    bool got = false;
+    for (int spin = 0; spin < kDfSpin && !got; ++spin) {
+      bool all = true;
+#pragma unroll
+      for (int dir = 0; dir < 3; ++dir)
+#pragma unroll
+        for (int q = 0; q < W; ++q)
+          if (w[dir][q] == kDfEmpty) w[dir][q] = df_load(mb + dir * 64 * W + q);
+#pragma unroll
+      for (int dir = 0; dir < 3; ++dir)
+#pragma unroll
+        for (int q = 0; q < W; ++q) all &= w[dir][q] != kDfEmpty;
+      got = __all(all);
+    }
+    // (never by the order of the tickets: this and every later sweep of the
+    // solve ends its systems as breakdowns, see k_dilu_df)
+    if (!got && lane == 0) {
+      a.scw[sys].status = ST_BREAK;
+      __hip_atomic_store(a.dfctl + DF_FAILED, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (int dir = 0; dir < 3; ++dir) {
+      if (!fok[dir]) continue;
+      __builtin_memcpy(&fv[dir], w[dir], sizeof(fv[dir]));
+#pragma unroll
+      for (int q = 0; q < W; ++q) df_store(mb + dir * 64 * W + q, kDfEmpty);
+    }
+  }
 #pragma unroll
   for (int dir = 0; dir < 3; ++dir) {   // one direction after another: a tile edge lies on two faces
-    const C2<T> w = FWD ? cmul(fd[dir], fv[dir]) : fv[dir];
+    const C2<T> w = (FWD && !DF) ? cmul(fd[dir], fv[dir]) : fv[dir];
     const T c = T(fc[dir]);
     C2<T> r = P[fq[dir]];
     r.x -= c * w.x;
@@ -274,10 +366,66 @@ __global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a) {
 #pragma unroll
   for (int u = 0; u < NU; ++u) P[sw_point(lane, skew, u)] = R[u];
   wave_sync();
+  if constexpr (DF) {
+    // the faces of the downstream neighbours first: w of the high layers
+    // (forward; those tiles are full in that direction), z of the low ones
+    const int nb[3] = {1, L.ntx, L.ntx * L.nty};
+    const int g0[3] = {gi0, gj0, gk0}, n[3] = {L.A, L.B, L.C};
+#pragma unroll
+    for (int dir = 0; dir < 3; ++dir) {
+      if (FWD ? g0[dir] + TX >= n[dir] : g0[dir] == 0) continue;   // uniform
+      const int t0 = FWD ? TX - 1 : 0;
+      const int ti = dir == 0 ? t0 : li0, tj = dir == 0 ? li0 : (dir == 1 ? t0 : lj0), tk = dir == 2 ? t0 : lj0;
+      if (!(ti < ex && tj < ey && tk < ez)) continue;
+      const int q = ti + TX * (tj + TX * tk);
+      const int tn = tself + (FWD ? nb[dir] : -nb[dir]);
+      df_put(a.mail + (int64_t(si) * a.dftiles + tn) * (kDfWords * W) + (dir * 64 + lane) * W,
+             FWD ? cmul(PD[q], P[q]) : P[q]);
+    }
+  }
   C2<T>* __restrict__ dst = a.out + o;
 #pragma unroll
   for (int u = 0; u < NU; ++u)
     if (col_ok && u < ez) dst[e0 + u * kst] = P[lane + 64 * u];
+}
+
+template <class T, class V, bool FWD>
+__global__ __launch_bounds__(64) void k_dilu_ro(DiluArgs<T, V> a) {
+  __shared__ RoLds<T, V, FWD, false> lds;
+  ro_tile<T, V, FWD, false>(a, lds, blockIdx.x);
+}
+
+// Every tile of the sweep in one launch.  A workgroup takes a ticket for its
+// NW items, so that the tiles start in level order whatever the order of
+// dispatch: what a tile waits for is held by waves that are already running,
+// and every wait ends.  A wave loads its tile's own data, polls its upstream
+// neighbours' faces, sweeps, and hands its own faces on before it stores the
+// tile.  Tickets one by one cost 24 ns an item (two atomics on one word), four
+// by four 6.  One system, FP64, per application: 100x100x60+10 449 us by tile
+// levels, 314 with NW = 1, 237 with NW = 4 (3.6 us a level); 40x40x30+10 157, 84,
+// 92; 16 systems at 100x100x60+10 1787 by levels, 1704 with NW = 4.
+template <class T, class V, bool FWD, int NW>
+__global__ __launch_bounds__(64 * NW) void k_dilu_df(DiluArgs<T, V> a) {
+  __shared__ RoLds<T, V, FWD, true> lds[NW];
+  __shared__ int s_ticket;
+  const int failed = a.dfctl[DF_FAILED];   // (of an earlier launch)
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (threadIdx.x == 0)
+    s_ticket = __hip_atomic_fetch_add(a.dfctl + DF_TICKET, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const int work = __builtin_amdgcn_readfirstlane(s_ticket) * NW + wv;
+  if (work < a.ntiles * a.nact) {
+    // a wait that gave up leaves words in the mailboxes: nothing is swept with them
+    if (failed == 0) ro_tile<T, V, FWD, true>(a, lds[wv], work);
+    else if ((threadIdx.x & 63) == 0) a.scw[a.act[work % a.nact]].status = ST_BREAK;
+  }
+  __syncthreads();
+  // the last workgroup done leaves the counters as it found them
+  if (threadIdx.x == 0 &&
+      __hip_atomic_fetch_add(a.dfctl + DF_DONE, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == int(gridDim.x) - 1) {
+    __hip_atomic_store(a.dfctl + DF_TICKET, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(a.dfctl + DF_DONE, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 // ------------------------------------------------- red-black tile ordering

@@ -167,6 +167,10 @@ struct mt_ctx {
   struct KTime { long long launches = 0; double ms = 0.0, bytes = 0.0; } kt[2];
   std::vector<hipEvent_t> tev;  // event pool
   int64_t nnz_stencil = -1;     // stored AAii couplings (cached)
+  // single-launch reference-ordered DILU sweeps (df_prepare)
+  unsigned long long* df_mail = nullptr;
+  int* df_ctl = nullptr;
+  int df_tiles = 0, df_sys = 0;   // tiles of the plan and active systems the mailboxes are laid out for
   unsigned char* scratch_dev = nullptr;  // this device's copy of `scratch`
 };
 
@@ -513,11 +517,13 @@ static int ensure_brick(mt_ctx* ctx, bool transpose) {
 }
 
 // ====================================================== preconditioner data
+static int df_prepare(mt_ctx* ctx, const TilePlan& tp, int nsys);
+
 // Inverse pivots (DILU) or inverse diagonal (Jacobi) per unique frequency.
 // The DILU pivots of the transposed operator are those of A^T's blocks.
 template <class T>
 static int build_dinv(mt_ctx* ctx, int pc, bool transpose, const std::vector<double>& freqs,
-                      C2<T>** out) {
+                      C2<T>** out, int nsys = 1) {
   const Grid& g = ctx->hop.g;
   const int nf = (int)freqs.size();
   std::string key = std::string("dinv") + (sizeof(T) == 8 ? "64" : "32");
@@ -536,6 +542,7 @@ static int build_dinv(mt_ctx* ctx, int pc, bool transpose, const std::vector<dou
   // level-scheduled sweep (PC_setup per frequency, as UpdateFreq does)
   const bool rb = pc == PCK_DILU_RB;
   const TilePlan& tp = rb ? ctx->tiles_rb : ctx->tiles;
+  if (!rb && (rc = df_prepare(ctx, tp, nsys))) return rc;
   double* dfreq;
   if ((rc = ws(ctx, "freqs", nf, &dfreq))) return rc;
   MT_HIP_CHECK(ctx, hipMemcpyAsync(dfreq, freqs.data(), nf * sizeof(double), hipMemcpyHostToDevice,
@@ -594,23 +601,67 @@ static DiluArgs<T, V> dilu_args(const TilePlan& tp, const V* coef, int64_t cstri
   return a;
 }
 
-template <class T, class V>
-static void dilu_fwd(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
-  for (int L = 0; L < tp.nlev; ++L) {
-    a.tiles = tp.tiles + tp.lvl_off[L];
-    a.ntiles = tp.lvl_off[L + 1] - tp.lvl_off[L];
-    k_dilu_ro<T, V, true><<<a.ntiles * a.nact, 64, 0, ctx->stream>>>(a);
-  }
+// Mailboxes and counters of the single-launch reference-ordered sweeps, for up
+// to nsys active systems on a tile plan; emptied here, at the start of every
+// solve (nothing is allocated where a chunk of iterations may be captured).
+constexpr int kDfSys = 16;     // active systems the mailboxes hold at most
+// items a launch takes tickets for one by one (40x40x30+10: 375 items 84 us an
+// application against 92 four by four, 750 items 97 against 95)
+constexpr int kDfOne = 600;
+static int df_prepare(mt_ctx* ctx, const TilePlan& tp, int nsys) {
+  ctx->df_tiles = 0;
+  ctx->df_sys = std::min(nsys, kDfSys);
+  const size_t words = size_t(ctx->df_sys) * tp.ntall * kDfWords * (sizeof(Z) / 8);
+  int rc;
+  if ((rc = ws(ctx, "df_mail", words, &ctx->df_mail)) || (rc = ws(ctx, "df_ctl", DF_NCTL, &ctx->df_ctl))) return rc;
+  k_df_clear<<<int(std::min<size_t>(2048, (words + 255) / 256)), 256, 0, ctx->stream>>>(ctx->df_mail, words,
+                                                                                       ctx->df_ctl);
+  MT_HIP_CHECK(ctx, hipGetLastError());
+  ctx->df_tiles = tp.ntall;
+  return MT_OK;
 }
 
+// After an entry point's sweeps: whether a wait gave up (its solve's results are void).
+static int df_check(mt_ctx* ctx) {
+  if (ctx->df_tiles == 0) return MT_OK;
+  int bad = 0;
+  MT_HIP_CHECK(ctx, hipMemcpyAsync(&bad, ctx->df_ctl + DF_FAILED, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  MT_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+  return bad ? mt_fail(ctx, MT_E_DEVICE, "a DILU sweep waited in vain for a neighbouring tile") : MT_OK;
+}
+
+// One launch for the whole sweep for up to kDfSys active systems (16 at
+// 100x100x60+10: 1704 us an application against 1787; beyond, the mailboxes
+// grow and the level launches fill the chip), else one launch per tile level.
+template <class T, class V, bool FWD>
+static void dilu_ro(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
+  if (a.nact <= ctx->df_sys && ctx->df_tiles == tp.ntall) {
+    a.tiles = tp.tiles;
+    a.ntiles = tp.ntall;
+    a.mail = ctx->df_mail;
+    a.dftiles = ctx->df_tiles;
+    a.dfctl = ctx->df_ctl;
+    a.scw = const_cast<SysScal*>(a.sc);
+    const int items = a.ntiles * a.nact;
+    if (items > kDfOne) k_dilu_df<T, V, FWD, 4><<<(items + 3) / 4, 256, 0, ctx->stream>>>(a);
+    else k_dilu_df<T, V, FWD, 1><<<items, 64, 0, ctx->stream>>>(a);
+    return;
+  }
+  for (int q = 0; q < tp.nlev; ++q) {
+    const int L = FWD ? q : tp.nlev - 1 - q;
+    a.tiles = tp.tiles + tp.lvl_off[L];
+    a.ntiles = tp.lvl_off[L + 1] - tp.lvl_off[L];
+    k_dilu_ro<T, V, FWD><<<a.ntiles * a.nact, 64, 0, ctx->stream>>>(a);
+  }
+}
+template <class T, class V>
+static void dilu_fwd(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
+  dilu_ro<T, V, true>(ctx, tp, a);
+}
 template <class T, class V>
 static void dilu_bwd(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
   a.in = a.out;
-  for (int L = tp.nlev - 1; L >= 0; --L) {
-    a.tiles = tp.tiles + tp.lvl_off[L];
-    a.ntiles = tp.lvl_off[L + 1] - tp.lvl_off[L];
-    k_dilu_ro<T, V, false><<<a.ntiles * a.nact, 64, 0, ctx->stream>>>(a);
-  }
+  dilu_ro<T, V, false>(ctx, tp, a);
 }
 
 // Red-black tile ordering: red forward, black forward+backward, red
@@ -1105,7 +1156,7 @@ static int solve_fp64(mt_ctx* ctx, int nsys, const double* omegas, Z* b, Z* x,
   a.x = x;
   a.b = b;
   C2<double>* dinv = nullptr;
-  if ((rc = build_dinv<double>(ctx, o.precond, tr, freqs, &dinv))) return rc;
+  if ((rc = build_dinv<double>(ctx, o.precond, tr, freqs, &dinv, nsys))) return rc;
   a.dinv = dinv;
   if (o.precond == PCK_DILU_RB) {
     DiluArgs<double, double> fa;
@@ -1244,7 +1295,7 @@ static int solve_mixed(mt_ctx* ctx, int nsys, const double* omegas, Z* b, Z* x,
     a.ppair = 2 * nI;
   }
   C2<float>* dinv = nullptr;
-  if ((rc = build_dinv<float>(ctx, o.precond, tr, freqs, &dinv))) return rc;
+  if ((rc = build_dinv<float>(ctx, o.precond, tr, freqs, &dinv, nsys))) return rc;
   if (bricks) {
     // the pivots of every frequency in brick order
     const int64_t nB = ctx->bk.g.nB;
@@ -1795,6 +1846,7 @@ int mt_precond_apply(mt_ctx* ctx, double omega, int precond, const mt_zdouble* x
     MT_HIP_CHECK(ctx, hipMemcpyAsync(dy, dx, sizeof(Z) * g.nE, hipMemcpyDeviceToDevice, ctx->stream));
   }
   MT_HIP_CHECK(ctx, hipGetLastError());
+  if (precond == MT_PC_DILU && (rc = df_check(ctx))) return rc;
   return download_padded(ctx, 1, dy, y, "io_tmp");
 }
 
@@ -2211,6 +2263,7 @@ int mt_divcor(mt_ctx* ctx, double omega, mt_zdouble* ei, const mt_zdouble* phi0,
   h.status = ST_RUN;
   MT_HIP_CHECK(ctx, hipMemcpyAsync(a.sc, &h, sizeof(h), hipMemcpyHostToDevice, ctx->stream));
   const int nb = a.G;
+  if ((rc = df_prepare(ctx, dc.tiles, 1))) return rc;
   k_divc<<<nb, BS, 0, ctx->stream>>>(a, a.b);
   k_pcg_init<<<nb, BS, 0, ctx->stream>>>(a);
   k_pcg_fin<PF_INIT><<<1, BS, 0, ctx->stream>>>(a);
@@ -2238,6 +2291,7 @@ int mt_divcor(mt_ctx* ctx, double omega, mt_zdouble* ei, const mt_zdouble* phi0,
   }
   k_grad_sub<<<1024, BS, 0, ctx->stream>>>(a, view<double>(ctx, false));
   MT_HIP_CHECK(ctx, hipGetLastError());
+  if ((rc = df_check(ctx))) return rc;
   if (niter) *niter = hs[0].iter;
   if (relres) *relres = hs[0].rnorm / hs[0].bnorm;
   return download_padded(ctx, 1, a.e, ei, "io_tmp");
@@ -2381,7 +2435,7 @@ int mt_bench_precond(mt_ctx* ctx, int nsys, int precision, int precond, int reps
   auto run = [&](auto tagT) -> int {
     using T = decltype(tagT);
     C2<T>* dinv;
-    int r2 = build_dinv<T>(ctx, precond, false, freqs, &dinv);
+    int r2 = build_dinv<T>(ctx, precond, false, freqs, &dinv, nsys);
     if (r2) return r2;
     C2<T>* vin;
     C2<T>* vout;
@@ -3230,6 +3284,7 @@ int mt_qmr(mt_ctx* ctx, double omega, const mt_zdouble* b, mt_zdouble* x, int ma
   *niter = iter;
   rerr[iter - 1] = double(float(rnormin / bnorm));
   *failed = fl;
+  if (E.pc && (rc = df_check(ctx))) return rc;
   if ((rc = download_padded(ctx, 1, X, x, "io_tmp"))) return rc;
   if (fl) return mt_fail(ctx, MT_E_BREAKDOWN, "mt_qmr: breakdown (rho, psi, delta, epsilon or beta = 0)");
   if (iter >= maxit) return mt_fail(ctx, MT_E_MAXIT, "mt_qmr: not converged within maxit");

@@ -300,3 +300,29 @@ def test_rhs_fwd_dev_matches_oracle(gpu_ctx):
         want = o.rhs_fwd(e[s])
         assert rel(b[s], want) <= 1e-13, s
         assert np.array_equal(x0[s], e[s][ei]), s
+
+
+@pytest.mark.parametrize("nsys", [1, 7, 18])
+def test_dilu_single_launch_sweeps(gpu_ctx, nsys):
+    """The reference-ordered sweeps in one launch with tickets taken one by one
+    (1 system: 108 tiles) and four by four (7 systems), and by tile levels (18
+    systems, past the mailboxes' 16, then in one launch as systems stop): FP64
+    batches against the oracle's BiCGStab, twice in a row (the counters and
+    mailboxes are left as they were found)."""
+    print(f"case dilu single launch nsys={nsys}", flush=True)
+    dx, dy, dz, nza, lc = small_problem(48, nx=26, ny=17, nzAir=5, nzEarth=12)
+    o = sp2oracle.Problem(dx, dy, dz, nza, lc)
+    gpu_ctx.assemble(dx, dy, dz, nza, lc)
+    rng = np.random.default_rng(8)
+    om = 2 * np.pi * np.repeat(10.0 ** np.linspace(-2, 2, (nsys + 1) // 2), 2)[:nsys]
+    B = rng.standard_normal((nsys, o.nInt)) + 1j * rng.standard_normal((nsys, o.nInt))
+    for _ in range(2):
+        X, st = gpu_ctx.solve_batch(om, B, tol=1e-10, maxit=2000, precision=mtsp2.PREC_FP64,
+                                    precond=mtsp2.PC_DILU, chunk=5)
+        assert all(s["status"] == 0 for s in st), st
+        for s in sorted({0, nsys // 2, nsys - 1}):
+            o.update_freq(om[s])
+            xo, info = o.bicg(B[s], np.zeros(o.nInt, complex), maxit=2000, tol=1e-10)
+            assert rel(X[s], xo) <= 1e-8, s
+            z = gpu_ctx.precond_apply(om[s], B[s], mtsp2.PC_DILU)
+            assert rel(z, o.pc_usolve(o.pc_lsolve(B[s]))) <= 1e-12, s
