@@ -65,8 +65,6 @@ struct TileShape {
   // couplings) are stored by slot, so a level's lanes read consecutive words.
   unsigned int rpts[kRbNP];
   unsigned short rslot[kRbNP];
-  // rpts by (hyperplane, lane): lane l's point of hyperplane h, or ~0u
-  unsigned int lpts[22][64];
 };
 
 struct LatticeInfo {

@@ -343,10 +343,6 @@ static int build_tile_plan(mt_ctx* ctx, TilePlan& tp, int nlat, const LatticeInf
   for (int h = 0; h < sh.nlev; ++h)
     if (sh.lvl[h + 1] - sh.lvl[h] > 64)
       return mt_fail(ctx, MT_E_STATE, "tile hyperplane wider than a wave");
-  if (tp.tx == 8 && tp.ty == 8 && tp.tz == 8)
-    for (int h = 0; h < sh.nlev; ++h)
-      for (int l = 0; l < 64; ++l)
-        sh.lpts[h][l] = sh.lvl[h] + l < sh.lvl[h + 1] ? sh.rpts[sh.lvl[h] + l] : 0xffffffffu;
 
   MT_HIP_CHECK(ctx, hipMalloc(&tp.tiles, sizeof(int4) * std::max<size_t>(1, flat.size())));
   MT_HIP_CHECK(ctx, hipMalloc(&tp.shape, sizeof(TileShape)));
