@@ -35,7 +35,8 @@ typedef double _Complex mt_zdouble;
 /* ---- status codes ---------------------------------------------------- */
 #define MT_OK 0
 #define MT_E_ARG 1        /* bad argument / size mismatch                     */
-#define MT_E_DEVICE 2     /* HIP runtime error                                 */
+#define MT_E_DEVICE 2     /* HIP runtime error, or a DILU sweep that gave up
+                             waiting for a neighbouring tile                   */
 #define MT_E_OOM 3        /* device allocation failed                          */
 #define MT_E_NAN_RHS 4    /* right-hand side contains NaN (solver.f90:1500)    */
 #define MT_E_BREAKDOWN 5  /* BiCGStab breakdown (alpha/beta/omega == 0)        */
@@ -77,7 +78,8 @@ typedef struct {
 typedef struct {
   int niter;            /* total BiCGStab iterations (inner for mixed)         */
   int nouter;           /* refinement steps (mixed) / true-residual rechecks   */
-  int status;           /* MT_OK, MT_E_BREAKDOWN, MT_E_MAXIT                   */
+  int status;           /* MT_OK, MT_E_BREAKDOWN, MT_E_MAXIT, MT_E_NAN_RHS,
+                           MT_E_DEVICE (mt_set_dilu_polls)                     */
   double relres;        /* final FP64 true relative residual                   */
 } mt_sys_stats;
 
@@ -396,6 +398,16 @@ int mt_set_spmv_variant(mt_ctx *ctx, int variant, int layers_per_segment);
  * operator; 5 and 6 round the black tiles' backward sweep differently from 1
  * and 4 (6 is bitwise 5).  No counterpart in the reference. */
 int mt_set_dilu_variant(mt_ctx *ctx, int variant);
+/* Polls a tile of the reference-ordered DILU (MT_PC_DILU), whose sweeps are one
+ * launch each for up to 16 active systems, spends waiting for its neighbours'
+ * faces before it gives up (default 65536, about 0.1 s; the tiles run in an
+ * order in which every wait ends).  Where one gives up, mt_solve_batch(_dev)
+ * return MT_E_DEVICE, with that status in the stats of the systems it ended
+ * (their x is void; systems that had stopped before keep theirs), and the
+ * other entry points that sweep return MT_E_DEVICE without their outputs.  0:
+ * every wait gives up at once, which is how that path is tested.  No
+ * counterpart in the reference. */
+int mt_set_dilu_polls(mt_ctx *ctx, int polls);
 /* Layout of the mixed solver's inner FP32 vectors when they are
  * preconditioned by the red-black DILU with the default SpMV: 2 (default) =
  * bricks (each 8x8x8 tile of the red-black plan contiguous) with the

@@ -124,6 +124,7 @@ struct DiluArgs {
   unsigned long long* mail = nullptr;
   int64_t dftiles = 0;     // tiles per active system in mail
   int* dfctl = nullptr;
+  int dfpolls = 0;         // polls before a wait gives up
   SysScal* scw = nullptr;
 };
 
@@ -136,7 +137,7 @@ struct DiluArgs {
 // kDfEmpty is a signalling NaN pattern that no arithmetic result has.
 constexpr unsigned long long kDfEmpty = 0xfff7a5a5fff7a5a5ull;
 constexpr int kDfWords = 3 * 64;          // complex entries per tile and active system
-constexpr int kDfSpin = 1 << 16;          // polls before a wait gives up (about 0.1 s)
+constexpr int kDfPolls = 1 << 16;         // polls before a wait gives up by default (about 0.1 s)
 // (a cache line each: the counters are atomics of every workgroup)
 enum : int { DF_TICKET = 0, DF_DONE = 64, DF_FAILED = 128, DF_NCTL = 192 };
 
@@ -307,7 +308,7 @@ __device__ __forceinline__ void ro_tile(const DiluArgs<T, V>& a, RoLds<T, V, FWD
 #pragma unroll
       for (int q = 0; q < W; ++q) w[dir][q] = fok[dir] ? kDfEmpty : 0;
     bool got = false;
-    for (int spin = 0; spin < kDfSpin && !got; ++spin) {
+    for (int n = 0; n < a.dfpolls && !got; ++n) {
       bool all = true;
 #pragma unroll
       for (int dir = 0; dir < 3; ++dir)
@@ -321,7 +322,8 @@ __device__ __forceinline__ void ro_tile(const DiluArgs<T, V>& a, RoLds<T, V, FWD
       got = __all(all);
     }
     // (never by the order of the tickets: this and every later sweep of the
-    // solve ends its systems as breakdowns, see k_dilu_df)
+    // entry point ends the systems that still run as breakdowns, see k_dilu_df,
+    // and the host returns MT_E_DEVICE, df_check)
     if (!got && lane == 0) {
       a.scw[sys].status = ST_BREAK;
       __hip_atomic_store(a.dfctl + DF_FAILED, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -415,7 +417,11 @@ __global__ __launch_bounds__(64 * NW) void k_dilu_df(DiluArgs<T, V> a) {
   if (work < a.ntiles * a.nact) {
     // a wait that gave up leaves words in the mailboxes: nothing is swept with them
     if (failed == 0) ro_tile<T, V, FWD, true>(a, lds[wv], work);
-    else if ((threadIdx.x & 63) == 0) a.scw[a.act[work % a.nact]].status = ST_BREAK;
+    else if ((threadIdx.x & 63) == 0) {
+      // (a system that has already stopped but is still in the list keeps its status)
+      SysScal& sc = a.scw[a.act[work % a.nact]];
+      if (sc.status == a.status_req) sc.status = ST_BREAK;
+    }
   }
   __syncthreads();
   // the last workgroup done leaves the counters as it found them

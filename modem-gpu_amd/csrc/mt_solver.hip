@@ -171,6 +171,7 @@ struct mt_ctx {
   unsigned long long* df_mail = nullptr;
   int* df_ctl = nullptr;
   int df_tiles = 0, df_sys = 0;   // tiles of the plan and active systems the mailboxes are laid out for
+  int df_polls = kDfPolls;        // mt_set_dilu_polls
   unsigned char* scratch_dev = nullptr;  // this device's copy of `scratch`
 };
 
@@ -617,7 +618,8 @@ static int df_prepare(mt_ctx* ctx, const TilePlan& tp, int nsys) {
   return MT_OK;
 }
 
-// After an entry point's sweeps: whether a wait gave up (its solve's results are void).
+// After an entry point's sweeps: MT_E_DEVICE if a wait gave up (what its systems
+// still running then have is void).
 static int df_check(mt_ctx* ctx) {
   if (ctx->df_tiles == 0) return MT_OK;
   int bad = 0;
@@ -637,6 +639,7 @@ static void dilu_ro(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
     a.mail = ctx->df_mail;
     a.dftiles = ctx->df_tiles;
     a.dfctl = ctx->df_ctl;
+    a.dfpolls = ctx->df_polls;
     a.scw = const_cast<SysScal*>(a.sc);
     const int items = a.ntiles * a.nact;
     if (items > kDfOne) k_dilu_df<T, V, FWD, 4><<<(items + 3) / 4, 256, 0, ctx->stream>>>(a);
@@ -1116,11 +1119,21 @@ static int compact(mt_ctx* ctx, const std::vector<SysScal>& h, int* d_act, std::
 }
 static bool keep_running(int st) { return st == ST_RUN || st == ST_RECHECK; }
 
+// df_check for a solve that left the records h: a sweep that gave up ended
+// its systems as breakdowns, so without one there is nothing to read.
+static int df_check_broken(mt_ctx* ctx, int pc, const std::vector<SysScal>& h) {
+  if (pc != PCK_DILU) return MT_OK;
+  for (const SysScal& s : h)
+    if (s.status == ST_BREAK) return df_check(ctx);
+  return MT_OK;
+}
+
 // FP64 BiCGStab on nsys padded systems (b, x device, system-major), the
 // semantics of cuBiCG.  Fills final SysScal records and the rerr history.
+// *swept: df_check's result (the records and x are filled either way).
 static int solve_fp64(mt_ctx* ctx, int nsys, const double* omegas, Z* b, Z* x,
                       const mt_solve_opts& o, std::vector<SysScal>& fin,
-                      std::vector<double>* rerr_out) {
+                      std::vector<double>* rerr_out, int* swept) {
   const Grid& g = ctx->hop.g;
   const int64_t nE = g.nE;
   const size_t nv = size_t(g.vlen(nsys));
@@ -1222,14 +1235,17 @@ static int solve_fp64(mt_ctx* ctx, int nsys, const double* omegas, Z* b, Z* x,
                                      hipMemcpyDeviceToHost, ctx->stream));
   }
   MT_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+  *swept = df_check_broken(ctx, o.precond, h);
   fin = h;
   return MT_OK;
 }
 
 // Mixed precision: FP32 BiCGStab inner solves inside FP64 defect correction.
+// *swept as for solve_fp64; a system that was refining then keeps its last
+// outer iterate and status ST_RUN.
 static int solve_mixed(mt_ctx* ctx, int nsys, const double* omegas, Z* b, Z* x,
                        const mt_solve_opts& o, std::vector<SysScal>& fin_out,
-                       std::vector<SysScal>* fin_in, std::vector<double>* rerr_out) {
+                       std::vector<SysScal>* fin_in, std::vector<double>* rerr_out, int* swept) {
   const Grid& g = ctx->hop.g;
   const int64_t nE = g.nE;
   const size_t nv = size_t(g.vlen(nsys));
@@ -1367,6 +1383,7 @@ static int solve_mixed(mt_ctx* ctx, int nsys, const double* omegas, Z* b, Z* x,
   MT_HIP_CHECK(ctx, hipGetLastError());
   if ((rc = read_scal(ctx, d_so, nsys, ho))) return rc;
   const int chunk = std::max(1, o.chunk);
+  *swept = MT_OK;
   while (true) {
     // outer: FP64 residual of the systems still refining
     const int n = compact(ctx, ho, d_act, act, [](int st) { return st == ST_RUN; });
@@ -1405,6 +1422,8 @@ static int solve_mixed(mt_ctx* ctx, int nsys, const double* omegas, Z* b, Z* x,
         if (a.ppair) E.set_pairs(iact);
       }
     }
+    // (an inner solve ended by a sweep that gave up has no correction to add)
+    if ((*swept = df_check_broken(ctx, o.precond, hi))) break;
     // x += d / scale on the systems that refined
     MT_HIP_CHECK(ctx, hipMemcpyAsync(d_act, outer_act.data(), outer_act.size() * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
     act = outer_act;
@@ -1681,7 +1700,9 @@ int mt_bicg(mt_ctx* ctx, double omega, const mt_zdouble* b, mt_zdouble* x, int m
   if ((rc = upload_padded(ctx, 1, b, db, "io_tmp")) || (rc = upload_padded(ctx, 1, x, dx, "io_tmp"))) return rc;
   std::vector<SysScal> fin;
   std::vector<double> hist;
-  if ((rc = solve_fp64(ctx, 1, &omega, db, dx, o, fin, rerr ? &hist : nullptr))) return rc;
+  int swept;
+  if ((rc = solve_fp64(ctx, 1, &omega, db, dx, o, fin, rerr ? &hist : nullptr, &swept))) return rc;
+  if (swept) return swept;
   const SysScal& s = fin[0];
   if (s.iter < 0) return mt_fail(ctx, MT_E_NAN_RHS, "right-hand side contains NaN");
   if ((rc = download_padded(ctx, 1, dx, x, "io_tmp"))) return rc;
@@ -1693,8 +1714,10 @@ int mt_bicg(mt_ctx* ctx, double omega, const mt_zdouble* b, mt_zdouble* x, int m
   return MT_OK;
 }
 
+// *swept: MT_OK, or MT_E_DEVICE where a sweep gave up waiting (x and stats are
+// filled; what the systems with that status have is void).
 static int solve_batch_common(mt_ctx* ctx, int nsys, const double* omegas, Z* db, Z* dx,
-                              const mt_solve_opts* opts, mt_sys_stats* stats) {
+                              const mt_solve_opts* opts, mt_sys_stats* stats, int* swept) {
   mt_solve_opts o;
   if (opts) o = *opts; else mt_default_opts(&o);
   if (o.maxit < 1 || nsys < 1 || nsys > 64) return mt_fail(ctx, MT_E_ARG, "solve: 1 <= nsys <= 64, maxit >= 1");
@@ -1703,27 +1726,22 @@ static int solve_batch_common(mt_ctx* ctx, int nsys, const double* omegas, Z* db
   if (o.precision != MT_PREC_FP64 && o.precision != MT_PREC_MIXED)
     return mt_fail(ctx, MT_E_ARG, "solve: unknown precision");
   std::vector<SysScal> fin;
+  const bool mixed = o.precision == MT_PREC_MIXED;
   int rc;
-  if (o.precision == MT_PREC_MIXED) {
+  if (mixed) {
     std::vector<SysScal> fin_in;
-    if ((rc = solve_mixed(ctx, nsys, omegas, db, dx, o, fin, &fin_in, nullptr))) return rc;
-    if (stats)
-      for (int s = 0; s < nsys; ++s) {
-        stats[s].niter = fin[s].tot_inner;
-        stats[s].nouter = fin[s].iter;
-        stats[s].status = fin[s].iter < 0 ? MT_E_NAN_RHS : status_code(fin[s].status);
-        stats[s].relres = fin[s].bnorm > 0 ? fin[s].rnorm / fin[s].bnorm : 0.0;
-      }
+    if ((rc = solve_mixed(ctx, nsys, omegas, db, dx, o, fin, &fin_in, nullptr, swept))) return rc;
   } else {
-    if ((rc = solve_fp64(ctx, nsys, omegas, db, dx, o, fin, nullptr))) return rc;
-    if (stats)
-      for (int s = 0; s < nsys; ++s) {
-        stats[s].niter = fin[s].iter;
-        stats[s].nouter = 0;
-        stats[s].status = fin[s].iter < 0 ? MT_E_NAN_RHS : status_code(fin[s].status);
-        stats[s].relres = fin[s].bnorm > 0 ? fin[s].rnorm / fin[s].bnorm : 0.0;
-      }
+    if ((rc = solve_fp64(ctx, nsys, omegas, db, dx, o, fin, nullptr, swept))) return rc;
   }
+  if (stats)
+    for (int s = 0; s < nsys; ++s) {
+      const bool ended = *swept && fin[s].status == (mixed ? ST_RUN : ST_BREAK);
+      stats[s].niter = mixed ? fin[s].tot_inner : fin[s].iter;
+      stats[s].nouter = mixed ? fin[s].iter : 0;
+      stats[s].status = fin[s].iter < 0 ? MT_E_NAN_RHS : (ended ? *swept : status_code(fin[s].status));
+      stats[s].relres = fin[s].bnorm > 0 ? fin[s].rnorm / fin[s].bnorm : 0.0;
+    }
   return MT_OK;
 }
 
@@ -1737,8 +1755,11 @@ int mt_solve_batch(mt_ctx* ctx, int nsys, const double* omegas, const mt_zdouble
   Z *db, *dx;
   if ((rc = ws(ctx, "io_b", g.vlen(nsys), &db)) || (rc = ws(ctx, "io_x", g.vlen(nsys), &dx))) return rc;
   if ((rc = upload_padded(ctx, nsys, b, db, "io_tmp")) || (rc = upload_padded(ctx, nsys, x, dx, "io_tmp"))) return rc;
-  if ((rc = solve_batch_common(ctx, nsys, omegas, db, dx, opts, stats))) return rc;
-  return download_padded(ctx, nsys, dx, x, "io_tmp");
+  int swept;
+  if ((rc = solve_batch_common(ctx, nsys, omegas, db, dx, opts, stats, &swept)) ||
+      (rc = download_padded(ctx, nsys, dx, x, "io_tmp")))
+    return rc;
+  return swept;
 }
 
 int mt_solve_batch_dev(mt_ctx* ctx, int nsys, const double* omegas, const void* b_dev, void* x_dev,
@@ -1755,11 +1776,12 @@ int mt_solve_batch_dev(mt_ctx* ctx, int nsys, const double* omegas, const void* 
   k_scatter<double, double><<<1024, 256, 0, ctx->stream>>>(ctx->dop.imap, g.nInt, g.nE, nsys, (const Z*)b_dev, db);
   k_scatter<double, double><<<1024, 256, 0, ctx->stream>>>(ctx->dop.imap, g.nInt, g.nE, nsys, (const Z*)x_dev, dx);
   MT_HIP_CHECK(ctx, hipGetLastError());
-  if ((rc = solve_batch_common(ctx, nsys, omegas, db, dx, opts, stats))) return rc;
+  int swept;
+  if ((rc = solve_batch_common(ctx, nsys, omegas, db, dx, opts, stats, &swept))) return rc;
   k_gather<double, double><<<1024, 256, 0, ctx->stream>>>(ctx->dop.imap, g.nInt, g.nE, nsys, dx, (Z*)x_dev);
   MT_HIP_CHECK(ctx, hipGetLastError());
   MT_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-  return MT_OK;
+  return swept;
 }
 
 int mt_dev_alloc(mt_ctx* ctx, size_t bytes, void** ptr) {
@@ -2473,6 +2495,7 @@ int mt_bench_precond(mt_ctx* ctx, int nsys, int precision, int precond, int reps
     MT_HIP_CHECK(ctx, hipEventRecord(ctx->ev[1], ctx->stream));
     MT_HIP_CHECK(ctx, hipEventSynchronize(ctx->ev[1]));
     MT_HIP_CHECK(ctx, hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
+    if (precond == MT_PC_DILU && (r2 = df_check(ctx))) return r2;
     if (bytes_per_apply)
       *bytes_per_apply = 6.0 * double(g.nInt) * sizeof(T) + double(nsys) * g.nInt * 3.0 * 2.0 * sizeof(T);
     return MT_OK;
@@ -2487,6 +2510,12 @@ int mt_set_dilu_variant(mt_ctx* ctx, int variant) {
   if (!ctx || (variant != 1 && variant != 4 && variant != 5 && variant != 6))
     return mt_fail(ctx, MT_E_ARG, "mt_set_dilu_variant: variant is 1, 4, 5 or 6");
   ctx->rb_variant = variant;
+  return MT_OK;
+}
+
+int mt_set_dilu_polls(mt_ctx* ctx, int polls) {
+  if (!ctx || polls < 0) return mt_fail(ctx, MT_E_ARG, "mt_set_dilu_polls: polls >= 0");
+  ctx->df_polls = polls;
   return MT_OK;
 }
 

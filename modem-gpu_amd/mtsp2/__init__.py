@@ -101,6 +101,7 @@ _SIGS = {
     "mt_timing_enable": (_I, [_P, _I]),
     "mt_set_spmv_variant": (_I, [_P, _I, _I]),
     "mt_set_dilu_variant": (_I, [_P, _I]),
+    "mt_set_dilu_polls": (_I, [_P, _I]),
     "mt_set_inner_layout": (_I, [_P, _I, _I]),
     "mt_inner_apply": (_I, [_P, _D, _I, _I, _PZ, _PZ]),
     "mt_bench_precond": (_I, [_P, _I, _I, _I, _I, C.POINTER(_D), C.POINTER(_D)]),
@@ -468,6 +469,11 @@ class Context:
         single-wave workgroup, 4 four systems per workgroup, 5 (default) four
         systems per workgroup in the lean LDS layout."""
         self._chk(lib().mt_set_dilu_variant(self._h, int(variant)))
+
+    def set_dilu_polls(self, polls):
+        """Polls before a tile of the single-launch reference-ordered DILU
+        sweeps gives up waiting (0: at once, MT_E_DEVICE)."""
+        self._chk(lib().mt_set_dilu_polls(self._h, int(polls)))
 
     def set_inner_layout(self, bricks, systems_per_block=0):
         """Inner FP32 vectors of the mixed solver (red-black DILU, default

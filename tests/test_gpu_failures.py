@@ -11,7 +11,10 @@ every kernel still ends normally:
                                         with a skew-symmetric coupling makes
                                         <rt, A p> = 0 at the first iteration of
                                         BiCGStab and <q, A p> = 0 for QMR
+  a DILU sweep that gives up waiting -> MT_E_DEVICE (a poll limit of 0)
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -98,3 +101,65 @@ def test_forced_breakdown(gpu_ctx):
     assert st[0]["status"] == mtsp2.MT_E_BREAKDOWN
     xq, nq, _, fq, sq = ctx.qmr(1.0, b, None, maxit=50, tol=1e-10, precond=mtsp2.PC_NONE)
     assert sq == mtsp2.MT_E_BREAKDOWN and fq
+
+
+def _raw_batch(ctx, om, B, **opts):
+    """mt_solve_batch's code, x and stats (the binding raises on the code)."""
+    om = np.ascontiguousarray(om, np.float64)
+    B = np.ascontiguousarray(B, np.complex128)
+    X = np.zeros_like(B)
+    st = (mtsp2.SysStats * len(om))()
+    o = mtsp2.default_opts(**opts)
+    rc = mtsp2.lib().mt_solve_batch(ctx._h, len(om), om, B, X, ctypes.byref(o), st)
+    return rc, X, [s.status for s in st]
+
+
+def test_dilu_wait_gives_up(gpu_ctx):
+    """A tile of a single-launch reference-ordered DILU sweep that gives up
+    waiting (forced: no polls at all): every entry point that sweeps returns
+    MT_E_DEVICE.  In a batch of 18 systems the sweeps run by tile levels until
+    two have converged and give up then: those keep their fields, the others
+    report MT_E_DEVICE.  Afterwards the same solves are what they were."""
+    print("case dilu wait gives up", flush=True)
+    dx, dy, dz, nza, lc = small_problem(48, nx=26, ny=17, nzAir=5, nzEarth=12)
+    ctx = gpu_ctx
+    ctx.assemble(dx, dy, dz, nza, lc)
+    n = ctx.n_int
+    rng = np.random.default_rng(9)
+    B = rng.standard_normal((18, n)) + 1j * rng.standard_normal((18, n))
+    om = 2 * np.pi * np.repeat(10.0 ** np.linspace(-2, 2, 9), 2)
+    fp64 = dict(tol=1e-9, maxit=2000, precond=mtsp2.PC_DILU, precision=mtsp2.PREC_FP64, chunk=3)
+    mixed = dict(fp64, precision=mtsp2.PREC_MIXED)
+    calls = {
+        "bicg": lambda: ctx.bicg(om[0], B[0], tol=1e-9),
+        "qmr": lambda: ctx.qmr(om[0], B[0], tol=1e-9),
+        "precond_apply": lambda: ctx.precond_apply(om[0], B[0]),
+        "divcor": lambda: ctx.divcor(om[0], B[0], tol=1e-6),
+        "bench_precond": lambda: ctx.bench_precond(2, mtsp2.PREC_FP64, mtsp2.PC_DILU, reps=1),
+    }
+    rc, X, st = _raw_batch(ctx, om, B, **fp64)
+    assert rc == 0 and not any(st)
+    z = ctx.precond_apply(om[0], B[0])
+    try:
+        ctx.set_dilu_polls(0)
+        for name, call in calls.items():
+            print("  ", name, flush=True)
+            with pytest.raises(mtsp2.MTError) as ei:
+                call()
+            assert ei.value.code == mtsp2.MT_E_DEVICE, name
+        for opts in (fp64, mixed):
+            rc, _, s = _raw_batch(ctx, om[:3], B[:3], **opts)
+            assert rc == mtsp2.MT_E_DEVICE and s == [mtsp2.MT_E_DEVICE] * 3, opts
+        rc, X0, s0 = _raw_batch(ctx, om, B, **fp64)
+        assert rc == mtsp2.MT_E_DEVICE
+        assert set(s0) == {mtsp2.MT_OK, mtsp2.MT_E_DEVICE}
+        done = [q for q in range(18) if s0[q] == mtsp2.MT_OK]
+        assert len(done) >= 2 and np.array_equal(X0[done], X[done])
+        # the red-black sweeps wait for nothing
+        rc, _, s = _raw_batch(ctx, om[:3], B[:3], **dict(mixed, precond=mtsp2.PC_DILU_RB))
+        assert rc == 0 and not any(s)
+    finally:
+        ctx.set_dilu_polls(1 << 16)   # the library's default
+    rc, X1, st = _raw_batch(ctx, om, B, **fp64)
+    assert rc == 0 and not any(st) and np.array_equal(X1, X)
+    assert np.array_equal(ctx.precond_apply(om[0], B[0]), z)
