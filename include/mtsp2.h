@@ -50,8 +50,8 @@ typedef double _Complex mt_zdouble;
 #define MT_PC_DILU 0      /* block diagonal-ILU, the reference's PC_setup      */
 #define MT_PC_JACOBI 1
 #define MT_PC_NONE 2
-#define MT_PC_DILU_RB 3   /* block DILU in red-black tile order: 2 launches per
-                             sweep instead of one per tile level; changes the
+#define MT_PC_DILU_RB 3   /* block DILU in red-black tile order: three launches
+                             per application, whatever the batch; changes the
                              iterates (not in the reference), meant for the
                              inner solves of MT_PREC_MIXED                    */
 #define MT_PREC_FP64 0
@@ -437,14 +437,15 @@ int mt_bench_spmv(mt_ctx *ctx, int nsys, int precision, int reps, double *ms_per
  * summed over every solve since the last mt_timing_enable (which resets it;
  * on = 0 turns the events off).  family MT_KT_SPMV: one event pair around each
  * fused SpMV+dot launch; MT_KT_PRECOND: one pair around each preconditioner
- * application (block DILU: one launch per tile level and sweep; red-black
- * tile DILU: three launches), so its time includes the gaps between those
- * launches.  launches: kernel launches covered; ms: summed event time; bytes:
- * algorithmic bytes of those launches (SpMV: stored couplings + diagonal per
- * launch, x, y and the dot partner per system; preconditioner: the six
- * lattice couplings per application, right-hand side(s), result and pivots
- * per system).  While timing is on, solves launch their kernels eagerly
- * (use_graph is ignored): HIP does not time events recorded by graph nodes. */
+ * application (block DILU: one launch per sweep for up to 16 active systems,
+ * else one per tile level and sweep; red-black tile DILU: three launches), so
+ * its time includes the gaps between those launches.  launches: kernel
+ * launches covered; ms: summed event time; bytes: algorithmic bytes of those
+ * launches (SpMV: stored couplings + diagonal per launch, x, y and the dot
+ * partner per system; preconditioner: the six lattice couplings per
+ * application, right-hand side(s), result and pivots per system).  While
+ * timing is on, solves launch their kernels eagerly (use_graph is ignored):
+ * HIP does not time events recorded by graph nodes. */
 #define MT_KT_SPMV 0
 #define MT_KT_PRECOND 1
 int mt_timing_enable(mt_ctx *ctx, int on);

@@ -631,8 +631,9 @@ static int df_check(mt_ctx* ctx) {
 // One launch for the whole sweep for up to kDfSys active systems (16 at
 // 100x100x60+10: 1704 us an application against 1787; beyond, the mailboxes
 // grow and the level launches fill the chip), else one launch per tile level.
+// Returns the number of launches, as every sweep function here does.
 template <class T, class V, bool FWD>
-static void dilu_ro(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
+static int dilu_ro(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
   if (a.nact <= ctx->df_sys && ctx->df_tiles == tp.ntall) {
     a.tiles = tp.tiles;
     a.ntiles = tp.ntall;
@@ -644,7 +645,7 @@ static void dilu_ro(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
     const int items = a.ntiles * a.nact;
     if (items > kDfOne) k_dilu_df<T, V, FWD, 4><<<(items + 3) / 4, 256, 0, ctx->stream>>>(a);
     else k_dilu_df<T, V, FWD, 1><<<items, 64, 0, ctx->stream>>>(a);
-    return;
+    return 1;
   }
   for (int q = 0; q < tp.nlev; ++q) {
     const int L = FWD ? q : tp.nlev - 1 - q;
@@ -652,15 +653,16 @@ static void dilu_ro(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
     a.ntiles = tp.lvl_off[L + 1] - tp.lvl_off[L];
     k_dilu_ro<T, V, FWD><<<a.ntiles * a.nact, 64, 0, ctx->stream>>>(a);
   }
+  return tp.nlev;
 }
 template <class T, class V>
-static void dilu_fwd(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
-  dilu_ro<T, V, true>(ctx, tp, a);
+static int dilu_fwd(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
+  return dilu_ro<T, V, true>(ctx, tp, a);
 }
 template <class T, class V>
-static void dilu_bwd(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
+static int dilu_bwd(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
   a.in = a.out;
-  dilu_ro<T, V, false>(ctx, tp, a);
+  return dilu_ro<T, V, false>(ctx, tp, a);
 }
 
 // Red-black tile ordering: red forward, black forward+backward, red
@@ -673,11 +675,12 @@ static int rb_grid(mt_ctx* ctx, int nwork) {
 }
 
 template <class T, class V>
-static void dilu_rb_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
+static int dilu_rb_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
   if (!a.xf) {  // every caller provides the packed-face buffer (rb_faces)
     ctx->err = "red-black DILU launched without its face buffer";
-    return;
+    return 0;
   }
+  int launches = 0;
   const int nl = tp.nlev;  // 2: red, black (a lattice of one tile has no black level)
   for (int step = 0; step < 3; ++step) {
     const int L = (step == 1) ? 1 : 0;
@@ -685,6 +688,7 @@ static void dilu_rb_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
     a.tiles = tp.tiles + tp.lvl_off[L];
     a.ntiles = tp.lvl_off[L + 1] - tp.lvl_off[L];
     if (a.ntiles == 0) continue;
+    ++launches;
     if (ctx->rb_variant >= 4) {
       constexpr int NW = 4;
       const int64_t nwork = int64_t(a.ntiles) * ((a.nact + NW - 1) / NW);
@@ -705,15 +709,17 @@ static void dilu_rb_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
     else if (step == 1) k_dilu_rb2<T, V, RB_BLACK_FB><<<g, 64, 0, ctx->stream>>>(a, tp.shape);
     else k_dilu_rb2<T, V, RB_RED_BWD><<<g, 64, 0, ctx->stream>>>(a, tp.shape);
   }
+  return launches;
 }
 
 // The red-black sweeps on bricks (k_dilu_bc): the three launches of
 // dilu_rb_apply, up to four systems of one tile per workgroup.
-static void dilu_bk_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<float, float> a) {
+static int dilu_bk_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<float, float> a) {
   if (!a.xf) {
     ctx->err = "red-black DILU launched without its face buffer";
-    return;
+    return 0;
   }
+  int launches = 0;
   // systems per workgroup: four share a tile's couplings; fewer active ones
   // take smaller workgroups instead of idle waves
   const int nw = a.nact >= 3 ? 4 : a.nact;
@@ -723,6 +729,7 @@ static void dilu_bk_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<float, float
     a.tiles = tp.tiles + tp.lvl_off[L];
     a.ntiles = tp.lvl_off[L + 1] - tp.lvl_off[L];
     if (a.ntiles == 0) continue;
+    ++launches;
     const int64_t nwork = int64_t(a.ntiles) * ((a.nact + nw - 1) / nw);
     const int g = int(8 * ((nwork + 7) / 8));
     // zp: the result pair-interleaved (zout: FP32 inner solves with paired x)
@@ -746,6 +753,7 @@ static void dilu_bk_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<float, float
     if (a.zout) launch_nw(std::true_type());
     else launch_nw(std::false_type());
   }
+  return launches;
 }
 
 // Packed i-face buffer of the red-black sweeps for systems 0..nsys-1
@@ -861,9 +869,9 @@ struct Engine {
     if (npair)
       hipMemcpyAsync(d_pairs, h_pairs.data(), npair * sizeof(int4), hipMemcpyHostToDevice, ctx->stream);
   }
-  // timing: event pairs (family, first, second) recorded by one chunk; with a
-  // graph they are recorded by the graph's event nodes on every replay
-  struct TPair { int fam, e0, e1; };
+  // timing: event pairs (family, first, second, kernel launches between them)
+  // recorded by one chunk
+  struct TPair { int fam, e0, e1, launches; };
   std::vector<TPair> tpairs;
   int tnext = 0;
   std::vector<int> last_iter;
@@ -872,13 +880,10 @@ struct Engine {
     hipEventRecord(ctx->tev[tnext], ctx->stream);
     return tnext++;
   }
-  void apply_pc(const DiluArgs<T, V>& d) {
-    if (a.pc == PCK_DILU_RB) {
-      dilu_rb_apply<T, V>(ctx, ctx->tiles_rb, d);
-    } else {
-      dilu_fwd<T, V>(ctx, ctx->tiles, d);
-      dilu_bwd<T, V>(ctx, ctx->tiles, d);
-    }
+  int apply_pc(const DiluArgs<T, V>& d) {
+    if (a.pc == PCK_DILU_RB) return dilu_rb_apply<T, V>(ctx, ctx->tiles_rb, d);
+    const int n = dilu_fwd<T, V>(ctx, ctx->tiles, d);
+    return n + dilu_bwd<T, V>(ctx, ctx->tiles, d);
   }
   // out = M^-1 (in - alpha*in2) (in2 may be null); with zout (bricks, paired
   // x) the result goes to zout pair-interleaved and out holds the red tiles'
@@ -907,9 +912,10 @@ struct Engine {
     d.xfsys = xfsys;
     d.xfhalf = xfhalf;
     const int e0 = ctx->timing ? trec() : -1;
-    if (!brick) apply_pc(d);
-    else if constexpr (sizeof(T) == 4) dilu_bk_apply(ctx, tp, d);
-    if (ctx->timing) tpairs.push_back({MT_KT_PRECOND, e0, trec()});
+    int launches = 0;
+    if (!brick) launches = apply_pc(d);
+    else if constexpr (sizeof(T) == 4) launches = dilu_bk_apply(ctx, tp, d);
+    if (ctx->timing) tpairs.push_back({MT_KT_PRECOND, e0, trec(), launches});
   }
   // the SpMV and its dot partials; returns the partial count per system
   template <int WHICH>
@@ -929,7 +935,7 @@ struct Engine {
           const int ngrp = (npair + spg - 1) / spg;
           k_spmv_btp<WHICH><<<b.G * ngrp, kBtThreads, 0, ctx->stream>>>(b, bg, bk_rows, d_pairs,
                                                                        npair, spg);
-          if (ctx->timing) tpairs.push_back({MT_KT_SPMV, e0, trec()});
+          if (ctx->timing) tpairs.push_back({MT_KT_SPMV, e0, trec(), 1});
           return b.G;
         }
       }
@@ -948,7 +954,7 @@ struct Engine {
       k_spmv_dot<T, V, WHICH><<<nblk, BS, 0, ctx->stream>>>(a);
       G = a.G;
     }
-    if (ctx->timing) tpairs.push_back({MT_KT_SPMV, e0, trec()});
+    if (ctx->timing) tpairs.push_back({MT_KT_SPMV, e0, trec(), 1});
     return G;
   }
 
@@ -1046,15 +1052,13 @@ struct Engine {
     }
     const Grid& g = ctx->hop.g;
     const double sv = sizeof(V), sc2 = 2.0 * sizeof(T), n = double(g.nInt);
-    const TilePlan& tp = a.pc == PCK_DILU_RB ? ctx->tiles_rb : ctx->tiles;
-    const int pc_launches = a.pc == PCK_DILU_RB ? 3 : 2 * tp.nlev;
     int cnt[2] = {0, 0};
     for (const TPair& tq : tpairs) {
       float ms = 0.f;
       MT_HIP_CHECK(ctx, hipEventElapsedTime(&ms, ctx->tev[tq.e0], ctx->tev[tq.e1]));
       mt_ctx::KTime& k = ctx->kt[tq.fam];
       k.ms += ms;
-      k.launches += tq.fam == MT_KT_SPMV ? 1 : pc_launches;
+      k.launches += tq.launches;
       ++cnt[tq.fam];
     }
     // SpMV, per launch: stored couplings + frequency-free diagonal; per system:

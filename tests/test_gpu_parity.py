@@ -178,6 +178,31 @@ def test_kernel_timing_graph_and_eager(gpu_ctx):
     assert gpu_ctx.kernel_timing(mtsp2.KT_SPMV) == (0, 0.0, 0.0)
 
 
+@pytest.mark.parametrize("nsys,precond,per_apply", [(2, mtsp2.PC_DILU, 2), (18, mtsp2.PC_DILU, None),
+                                                   (2, mtsp2.PC_DILU_RB, 3)])
+def test_kernel_timing_counts_launches(gpu_ctx, nsys, precond, per_apply):
+    """Kernel timing counts the launches there are: per preconditioner
+    application (as many as SpMV launches) one per sweep for up to 16 systems,
+    one per tile level ti+tj+tk of the interior edges' 8x8x8 tiles and sweep
+    beyond, three for the red-black ordering."""
+    print(f"case kernel timing counts nsys={nsys} precond={precond}", flush=True)
+    o, g = _setup(gpu_ctx, 7, nx=26, ny=17, nzAir=5, nzEarth=12)
+    rng = np.random.default_rng(10)
+    om = 2 * np.pi * np.linspace(0.1, 10.0, nsys)
+    B = rng.standard_normal((nsys, o.nInt)) + 1j * rng.standard_normal((nsys, o.nInt))
+    gpu_ctx.timing_enable(True)
+    try:
+        # (three iterations, no system done by then)
+        gpu_ctx.solve_batch(om, B, tol=1e-12, maxit=3, chunk=3, precision=mtsp2.PREC_FP64, precond=precond)
+        (spmv, _, _), (pc, ms, _) = [gpu_ctx.kernel_timing(f) for f in (mtsp2.KT_SPMV, mtsp2.KT_PRECOND)]
+    finally:
+        gpu_ctx.timing_enable(False)
+    assert spmv == 6 and ms > 0
+    n = (26, 17, 17)
+    levels = max(sum((n[d] - (d != c) + 7) // 8 - 1 for d in range(3)) for c in range(3)) + 1
+    assert pc == spmv * (per_apply or 2 * levels)
+
+
 @pytest.fixture
 def dilu_variant(gpu_ctx, request):
     """Launch shape of the red-black DILU for one test (restored after)."""
