@@ -131,11 +131,27 @@ struct DiluArgs {
 // ------------------------------------ faces in transit between running tiles
 // A tile hands its facing layer to its downstream neighbour through a mailbox
 // of its own: [active system][tile][direction][64 entries] complex, every
-// 8-byte word either a value or kDfEmpty, written and polled word by word with
+// 8-byte word either a value or df_empty, written and polled word by word with
 // relaxed agent-scope atomics (coherent across the XCDs; no fence, whose
 // write-back of an L2 costs microseconds).  The one reader empties it again.
-// kDfEmpty is a signalling NaN pattern that no arithmetic result has.
-constexpr unsigned long long kDfEmpty = 0xfff7a5a5fff7a5a5ull;
+// df_empty is a signalling NaN of the type T of the values, one double or two
+// floats to a word: what is handed on is the result of an arithmetic
+// instruction, and those return no signalling NaN, whatever NaN they are given.
+// (No word is one in both readings: a double's exponent covers the bit that
+// tells a float's quiet NaN.)
+template <class T>
+__host__ __device__ constexpr unsigned long long df_empty() {
+  return sizeof(T) == 8 ? 0xfff7a5a5fff7a5a5ull : 0xffb7a5a5ffb7a5a5ull;
+}
+constexpr bool df_signals64(unsigned long long w) {
+  return ((w >> 52) & 0x7ff) == 0x7ff && !((w >> 51) & 1) && (w & ((1ull << 51) - 1));
+}
+constexpr bool df_signals32(unsigned w) {
+  return ((w >> 23) & 0xff) == 0xff && !((w >> 22) & 1) && (w & ((1u << 22) - 1));
+}
+static_assert(df_signals64(df_empty<double>()) && df_signals32(unsigned(df_empty<float>())) &&
+                  df_signals32(unsigned(df_empty<float>() >> 32)),
+              "the mark of an empty word is a signalling NaN");
 constexpr int kDfWords = 3 * 64;          // complex entries per tile and active system
 constexpr int kDfPolls = 1 << 16;         // polls before a wait gives up by default (about 0.1 s)
 // (a cache line each: the counters are atomics of every workgroup)
@@ -155,10 +171,10 @@ __device__ __forceinline__ void df_put(unsigned long long* p, C2<T> v) {
 #pragma unroll
   for (int q = 0; q < W; ++q) df_store(p + q, w[q]);
 }
-// all of the words of the mailboxes empty, the counters zero
-__global__ void k_df_clear(unsigned long long* mail, int64_t n, int* ctl) {
+// all of the words of the mailboxes `empty`, the counters zero
+__global__ void k_df_clear(unsigned long long* mail, int64_t n, unsigned long long empty, int* ctl) {
   for (int64_t q = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; q < n; q += int64_t(gridDim.x) * blockDim.x)
-    mail[q] = kDfEmpty;
+    mail[q] = empty;
   if (blockIdx.x == 0 && threadIdx.x < DF_NCTL) ctl[threadIdx.x] = 0;
 }
 
@@ -301,12 +317,13 @@ __device__ __forceinline__ void ro_tile(const DiluArgs<T, V>& a, RoLds<T, V, FWD
   const int tself = L.tbase + tl.y + L.ntx * (tl.z + L.nty * tl.w);
   constexpr int W = sizeof(C2<T>) / 8;
   if constexpr (DF) {
+    constexpr unsigned long long kEmpty = df_empty<T>();
     unsigned long long* mb = a.mail + (int64_t(si) * a.dftiles + tself) * (kDfWords * W) + lane * W;
     unsigned long long w[3][W];
 #pragma unroll
     for (int dir = 0; dir < 3; ++dir)
 #pragma unroll
-      for (int q = 0; q < W; ++q) w[dir][q] = fok[dir] ? kDfEmpty : 0;
+      for (int q = 0; q < W; ++q) w[dir][q] = fok[dir] ? kEmpty : 0;
     bool got = false;
     for (int n = 0; n < a.dfpolls && !got; ++n) {
       bool all = true;
@@ -314,11 +331,11 @@ __device__ __forceinline__ void ro_tile(const DiluArgs<T, V>& a, RoLds<T, V, FWD
       for (int dir = 0; dir < 3; ++dir)
 #pragma unroll
         for (int q = 0; q < W; ++q)
-          if (w[dir][q] == kDfEmpty) w[dir][q] = df_load(mb + dir * 64 * W + q);
+          if (w[dir][q] == kEmpty) w[dir][q] = df_load(mb + dir * 64 * W + q);
 #pragma unroll
       for (int dir = 0; dir < 3; ++dir)
 #pragma unroll
-        for (int q = 0; q < W; ++q) all &= w[dir][q] != kDfEmpty;
+        for (int q = 0; q < W; ++q) all &= w[dir][q] != kEmpty;
       got = __all(all);
     }
     // (never by the order of the tickets: this and every later sweep of the
@@ -333,7 +350,7 @@ __device__ __forceinline__ void ro_tile(const DiluArgs<T, V>& a, RoLds<T, V, FWD
       if (!fok[dir]) continue;
       __builtin_memcpy(&fv[dir], w[dir], sizeof(fv[dir]));
 #pragma unroll
-      for (int q = 0; q < W; ++q) df_store(mb + dir * 64 * W + q, kDfEmpty);
+      for (int q = 0; q < W; ++q) df_store(mb + dir * 64 * W + q, kEmpty);
     }
   }
 #pragma unroll

@@ -514,6 +514,7 @@ static int ensure_brick(mt_ctx* ctx, bool transpose) {
 }
 
 // ====================================================== preconditioner data
+template <class T>
 static int df_prepare(mt_ctx* ctx, const TilePlan& tp, int nsys);
 
 // Inverse pivots (DILU) or inverse diagonal (Jacobi) per unique frequency.
@@ -539,7 +540,7 @@ static int build_dinv(mt_ctx* ctx, int pc, bool transpose, const std::vector<dou
   // level-scheduled sweep (PC_setup per frequency, as UpdateFreq does)
   const bool rb = pc == PCK_DILU_RB;
   const TilePlan& tp = rb ? ctx->tiles_rb : ctx->tiles;
-  if (!rb && (rc = df_prepare(ctx, tp, nsys))) return rc;
+  if (!rb && (rc = df_prepare<T>(ctx, tp, nsys))) return rc;
   double* dfreq;
   if ((rc = ws(ctx, "freqs", nf, &dfreq))) return rc;
   MT_HIP_CHECK(ctx, hipMemcpyAsync(dfreq, freqs.data(), nf * sizeof(double), hipMemcpyHostToDevice,
@@ -598,21 +599,22 @@ static DiluArgs<T, V> dilu_args(const TilePlan& tp, const V* coef, int64_t cstri
   return a;
 }
 
-// Mailboxes and counters of the single-launch reference-ordered sweeps, for up
-// to nsys active systems on a tile plan; emptied here, at the start of every
+// Mailboxes and counters of the single-launch reference-ordered sweeps in T, for
+// up to nsys active systems on a tile plan; emptied here, at the start of every
 // solve (nothing is allocated where a chunk of iterations may be captured).
 constexpr int kDfSys = 16;     // active systems the mailboxes hold at most
 // items a launch takes tickets for one by one (40x40x30+10: 375 items 84 us an
 // application against 92 four by four, 750 items 97 against 95)
 constexpr int kDfOne = 600;
+template <class T>
 static int df_prepare(mt_ctx* ctx, const TilePlan& tp, int nsys) {
   ctx->df_tiles = 0;
   ctx->df_sys = std::min(nsys, kDfSys);
-  const size_t words = size_t(ctx->df_sys) * tp.ntall * kDfWords * (sizeof(Z) / 8);
+  const size_t words = size_t(ctx->df_sys) * tp.ntall * kDfWords * (sizeof(C2<T>) / 8);
   int rc;
   if ((rc = ws(ctx, "df_mail", words, &ctx->df_mail)) || (rc = ws(ctx, "df_ctl", DF_NCTL, &ctx->df_ctl))) return rc;
   k_df_clear<<<int(std::min<size_t>(2048, (words + 255) / 256)), 256, 0, ctx->stream>>>(ctx->df_mail, words,
-                                                                                       ctx->df_ctl);
+                                                                                       df_empty<T>(), ctx->df_ctl);
   MT_HIP_CHECK(ctx, hipGetLastError());
   ctx->df_tiles = tp.ntall;
   return MT_OK;
@@ -2285,7 +2287,7 @@ int mt_divcor(mt_ctx* ctx, double omega, mt_zdouble* ei, const mt_zdouble* phi0,
   h.status = ST_RUN;
   MT_HIP_CHECK(ctx, hipMemcpyAsync(a.sc, &h, sizeof(h), hipMemcpyHostToDevice, ctx->stream));
   const int nb = a.G;
-  if ((rc = df_prepare(ctx, dc.tiles, 1))) return rc;
+  if ((rc = df_prepare<double>(ctx, dc.tiles, 1))) return rc;
   k_divc<<<nb, BS, 0, ctx->stream>>>(a, a.b);
   k_pcg_init<<<nb, BS, 0, ctx->stream>>>(a);
   k_pcg_fin<PF_INIT><<<1, BS, 0, ctx->stream>>>(a);

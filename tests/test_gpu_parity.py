@@ -351,3 +351,22 @@ def test_dilu_single_launch_sweeps(gpu_ctx, nsys):
             assert rel(X[s], xo) <= 1e-8, s
             z = gpu_ctx.precond_apply(om[s], B[s], mtsp2.PC_DILU)
             assert rel(z, o.pc_usolve(o.pc_lsolve(B[s]))) <= 1e-12, s
+
+
+def test_dilu_single_launch_nan(gpu_ctx):
+    """NaNs in the vector, the bit pattern that marks an empty mailbox word
+    among them, are handed from tile to tile like any value (an arithmetic
+    result is never that pattern): the application ends, without MT_E_DEVICE,
+    with NaN wherever the oracle has one."""
+    print("case dilu single launch NaN", flush=True)
+    o, g = _setup(gpu_ctx, 49, nx=26, ny=17, nzAir=5, nzEarth=12)
+    w = 2 * np.pi * 0.3
+    o.update_freq(w)
+    mark = np.array([0xfff7a5a5fff7a5a5], np.uint64).view(np.float64)[0]
+    for at in (slice(None), slice(0, None, 97)):
+        x = np.ones(o.nInt, complex)
+        x.view(np.float64)[np.arange(2 * o.nInt)[at]] = mark
+        z = gpu_ctx.precond_apply(w, x, mtsp2.PC_DILU)
+        want = o.pc_usolve(o.pc_lsolve(x))
+        assert np.isnan(want).any()
+        assert np.isnan(z)[np.isnan(want)].all()
