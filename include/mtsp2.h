@@ -219,10 +219,12 @@ int mt_rhs_fwd_dev(mt_ctx *ctx, int nsys, const void *e_dev, void *b_dev, void *
  * the bottom-face x and y edges zero), ready for mt_rhs_fwd_dev.  Equal to
  * the reference's fields bit for bit while its partial pivoting keeps the
  * diagonal; MT_E_PIVOT (fields still written) where it would not.
- * Needs nz <= about 100 (the slice window).  Scratch, kept by the context: the
- * rows of U of the slices in flight, up to 4*CUs*(nh-1)*(nz-1)*nz complex
- * doubles (6.7 GB at 100x100x70 on 256 CUs; fewer slices in flight where that
- * does not fit). */
+ * nz <= 100 (the slice window), else MT_E_ARG.  Scratch, kept by the context:
+ * for each slice in flight the rows of U, padded to nz' = 16*ceil(nz/16)
+ * entries, the right-hand side and the coefficients, (nh-1)*(nz-1)*(nz'+4)
+ * complex doubles.  As many slices are in flight as are resident at once, 4
+ * per CU for nz <= 64, 3 to 80, 2 to 96, else 1 (7.1 GB at 100x100x70 on 256
+ * CUs; fewer where that does not fit). */
 int mt_bc_x0_dev(mt_ctx *ctx, int nsys, const double *omegas, const int *modes, void *e_dev);
 /* Transposed (adjoint) RHS of FWDsolve3D's TRN branch with a dense source
  * (EMsolve3D.f90:217-256): b = s_i + V_E GDii(s_i (i*ISIGN*omega*mu0)^-1 / V_E),

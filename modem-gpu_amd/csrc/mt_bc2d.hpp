@@ -308,12 +308,8 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Largest nz the slices are taken at (an (nz x nz) window of complex doubles
-// and its staging within 160 KB).
-__host__ __device__ inline size_t bc_window_bytes(int nz) {
-  const size_t B1 = size_t(nz);
-  return (B1 * B1 + B1 + 65) * sizeof(double2) + 64 * sizeof(double);
-}
+// Largest nz mt_bc_x0_dev takes (the largest window, 16 x 7 slots, would hold 112).
+constexpr int kBcMaxNz = 100;
 
 // The arguments as if met for the first time: what one phase of a slice reads
 // of them is not kept in registers over the others.

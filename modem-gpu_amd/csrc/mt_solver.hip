@@ -1493,8 +1493,7 @@ static int download_padded(mt_ctx* ctx, int nsys, const Z* d, mt_zdouble* h, con
   return MT_OK;
 }
 
-// The slice kernel for nz: the smallest register window that holds it (the
-// entry point takes nz to about 100).
+// The slice kernel for nz: the smallest register window that holds it.
 struct BcKernel { const void* f; int threads, slots; };
 template <int TG, int R>
 static BcKernel bc_shape() {
@@ -1506,6 +1505,7 @@ static BcKernel bc_kernel(int nz) {
   if (nz <= 64) return bc_shape<16, 4>();
   if (nz <= 80) return bc_shape<16, 5>();
   if (nz <= 96) return bc_shape<16, 6>();
+  static_assert(kBcMaxNz <= 16 * 7, "a window that holds every nz taken");
   return bc_shape<16, 7>();
 }
 
@@ -2021,10 +2021,7 @@ int mt_bc_x0_dev(mt_ctx* ctx, int nsys, const double* omegas, const int* modes, 
     if ((modes[s] != 1 && modes[s] != 2) || !(omegas[s] > 0.0))
       return mt_fail(ctx, MT_E_ARG, "mt_bc_x0_dev: mode must be 1 or 2 and omega > 0");
   MT_HIP_CHECK(ctx, hipSetDevice(ctx->device));
-  int maxlds = 0;
-  MT_HIP_CHECK(ctx, hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device));
-  if (bc_window_bytes(nz) + 64 > size_t(maxlds) || nz > 112)
-    return mt_fail(ctx, MT_E_ARG, "mt_bc_x0_dev: nz too large for the slice window");
+  if (nz > kBcMaxNz) return mt_fail(ctx, MT_E_ARG, "mt_bc_x0_dev: nz too large for the slice window");
   const BcKernel bk = bc_kernel(nz);
   // host side: earth conductivities as ModelParamToCell forms them, block distances, items
   const int64_t nce = int64_t(nx) * ny * H.nzEarth;

@@ -123,8 +123,8 @@ def test_bc_x0_dev_full_size(gpu_ctx):
 
 
 def test_bc_x0_dev_deep_window(gpu_ctx):
-    """nz = 90 (the 120x120x80+10 configuration's depth): the band window
-    takes 131 KB of LDS, one slice per CU; bit for bit against the oracle."""
+    """nz = 90 (the 120x120x80+10 configuration's depth), two slices per CU;
+    bit for bit against the oracle."""
     print("case bc_x0 nz=90", flush=True)
     grid = P.make_grid(5, 4, 80, nair=10, npad=2)
     lc = P.boxes_model(grid, nbox=6, seed=8)
@@ -150,6 +150,16 @@ def test_bc_x0_dev_argument_errors(gpu_ctx):
         with pytest.raises(mtsp2.MTError) as ei:
             ctx.bc_x0(np.array(om), np.array(md))
         assert ei.value.code == mtsp2.MT_E_ARG
+
+
+def test_bc_x0_dev_depth_limit(gpu_ctx):
+    """nz = 101 is refused (nz = 100: test_bc_x0_dev_window_edges)."""
+    print("case bc_x0 nz=101", flush=True)
+    import mtsp2
+    gpu_ctx.assemble(np.full(3, 300.0), np.full(3, 300.0), np.full(101, 100.0), 20, np.full((3, 3, 81), -4.0))
+    with pytest.raises(mtsp2.MTError) as ei:
+        gpu_ctx.bc_x0(np.array([1.0]), np.array([1]))
+    assert ei.value.code == mtsp2.MT_E_ARG
 
 
 @pytest.mark.parametrize("nz", [3, 32, 33, 48, 49, 64, 65, 80, 81, 96, 97, 100])
