@@ -69,30 +69,43 @@ def test_brick_dilu_inverts_its_factorisation(gpu_ctx, transpose):
             assert rel(z, z64) <= 2e-5, f
 
 
-def test_brick_dilu_persistent_matches(gpu_ctx):
-    """The persistent brick DILU launches (variant 6: a workgroup walks its
-    items and loads the next one while it sweeps) do k_dilu_bk's arithmetic:
-    one application and batched solves are bitwise equal."""
-    print("case brick dilu persistent", flush=True)
+@pytest.mark.parametrize("transpose", [False, True])
+def test_brick_dilu_batches_match_single_systems(gpu_ctx, transpose):
+    """The brick DILU's workgroups of one, two and four waves (1, 2, 3 and 5
+    systems: 3 and 5 leave waves idle) and its sweeps with the p-update folded
+    in (variant 6) or run apart (5) are the same arithmetic per system.  With
+    the row chunks fixed, so that no sum's order depends on the batch, every
+    system's solve in every batch and variant is bitwise its solve alone with
+    the p-update apart (whose application test_brick_dilu_inverts_... and
+    test_brick_dilu_tile_edges check); the true residual by the FP64 apply."""
+    print(f"case brick dilu batches transpose={transpose}", flush=True)
     o, g = _grid(gpu_ctx, 44)
     grid = {"dx": g[0], "dy": g[1], "dz": g[2], "nzAir": g[3]}
-    rng = np.random.default_rng(6)
-    x = rng.standard_normal(o.nInt) + 1j * rng.standard_normal(o.nInt)
     om, B, X0 = P.forward_systems(gpu_ctx, grid, [1e-2, 0.5, 20.0])
-    res = {}
+
+    def solve(s):
+        X, st = gpu_ctx.solve_batch(om[s], B[s], X0[s], tol=1e-10, maxit=4000, precision=mtsp2.PREC_MIXED,
+                                    precond=mtsp2.PC_DILU_RB, op_transpose=int(transpose))
+        return X, [(q["status"], q["niter"], q["nouter"]) for q in st]
+
     try:
+        gpu_ctx.set_tuning(64)
+        gpu_ctx.set_dilu_variant(5)
+        alone = [solve(slice(s, s + 1)) for s in range(5)]
+        for s, (X, st) in enumerate(alone):
+            assert st[0][0] == 0
+            r = B[s] - gpu_ctx.apply(om[s], X[0], transpose=int(transpose))
+            assert np.linalg.norm(r) <= 1e-10 * 1.0001 * np.linalg.norm(B[s]), s
         for v in (5, 6):
             gpu_ctx.set_dilu_variant(v)
-            z = [gpu_ctx.inner_apply(2 * np.pi * 0.7, x, what=1, transpose=t) for t in (False, True)]
-            X, st = gpu_ctx.solve_batch(om, B, X0, tol=1e-10, maxit=4000, precision=mtsp2.PREC_MIXED,
-                                        precond=mtsp2.PC_DILU_RB)
-            res[v] = (z, X, [(s["niter"], s["nouter"]) for s in st])
+            for n in (1, 2, 3, 5):
+                X, st = solve(slice(0, n))
+                for s in range(n):
+                    assert st[s] == alone[s][1][0], (v, n, s)
+                    assert np.array_equal(X[s], alone[s][0][0]), (v, n, s)
     finally:
-        gpu_ctx.set_dilu_variant(6)   # the library's default
-    for t in range(2):
-        assert np.array_equal(res[5][0][t], res[6][0][t]), t
-    assert res[5][2] == res[6][2]
-    assert np.array_equal(res[5][1], res[6][1])
+        gpu_ctx.set_dilu_variant(6)   # the library's defaults
+        gpu_ctx.set_tuning(0)
 
 
 @pytest.mark.parametrize("transpose,nsys", [(False, 5), (True, 5), (False, 1)])
