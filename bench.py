@@ -446,7 +446,7 @@ def main():
     if on_bricks:
         rb_kernel = ("k_dilu_bc<float,float,RED_FWD|BLACK_FB|RED_BWD,4> (on bricks, tiles swept in "
                      "registers)")
-    pc_kernels = {0: "k_dilu_tile<float,float,8,8,8,true|false> (block-DILU level sweeps)",
+    pc_kernels = {0: "k_dilu_df|k_dilu_ro<float,float,true|false> (reference-ordered block-DILU sweeps)",
                   3: rb_kernel + " (red-black tile block-DILU, 3 launches per application)"}
     spv = 3 if args.spmv_variant is None else args.spmv_variant
     spmv_kernels = {0: "k_spmv_dot<float,float,1|2> (row-parallel v = A x with its dot products)",

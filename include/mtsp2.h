@@ -424,7 +424,10 @@ int mt_set_inner_layout(mt_ctx *ctx, int bricks, int systems_per_block);
 /* The inner solves' brick kernels on one vector, for checking them: y = A x
  * (what = 0) or y = M^-1 x (what = 1, the red-black DILU of A(omega)), of A
  * (transpose = 0) or A^T (1), computed in FP32 on bricks; x, y: n_int
- * complex in EDGEi order.  No counterpart in the reference. */
+ * complex in EDGEi order.  x finite: with what = 1 a NaN or an infinity spoils
+ * the whole of its tile and of the tiles around it, points that do not depend
+ * on it among them (in a solve its system ends as a breakdown).  No counterpart
+ * in the reference. */
 int mt_inner_apply(mt_ctx *ctx, double omega, int what, int transpose, const mt_zdouble *x,
                    mt_zdouble *y);
 /* Fixes the row-tile group count per system (0: automatic). */

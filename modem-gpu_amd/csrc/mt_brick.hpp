@@ -506,8 +506,8 @@ __global__ __launch_bounds__(kBtThreads, 4) void k_spmv_btp(IterArgs<float, floa
 // DiluArgs on bricks: coef = the [6][nB] couplings (slots 1..6), cstride =
 // nB, vstride = nB, dinv = [nfreq][nB].
 // What bounds it: memory at many systems (100x100x60+10, 16 systems: red
-// forward 404 MB in 89 us, black 567 MB in 132 us, red backward 511 MB in 108
-// us, 4.3-4.7 TB/s of a copy's 4.9-5.4; per application 327 us, where sweeps
+// forward 404 MB in 94 us, black 568 MB in 132 us, red backward 511 MB in 106
+// us, 4.3-4.8 TB/s of a copy's 4.9-5.4; per application 330 us, where sweeps
 // out of an LDS box took 461 with persistent workgroups that loaded their next
 // tile meanwhile), one tile's chain of loads, sweep and stores at few (two
 // systems 56 us against 116; 40x40x30+10 19 against 41).  The sweeps are short

@@ -9,12 +9,14 @@
 // 2055) are solved by wavefronts over the hyperplanes i+j+k = const.
 //
 // Instead of one launch per hyperplane (266 at 100x100x60+10), the lattice is
-// cut into TX*TY*TZ tiles.  One launch handles every tile of one tile-level
-// ti+tj+tk = L (all three blocks and all active systems at once); inside a
-// tile one wave64 sweeps the tile's own hyperplanes out of LDS, with the
-// upstream faces (final after the previous launch) staged into an LDS halo.
-// Launch boundaries are the only inter-tile synchronisation, so nothing ever
-// spins on a flag.
+// cut into 8x8x8 tiles, swept by one wave64 each in registers (mt_sweep.hpp;
+// the red-black sweeps of the all-edge layout, k_dilu_rb2/rbm/rbl, out of LDS),
+// for all three blocks and all active systems at once.  In the reference's
+// ordering a tile depends on its low (backward: high) neighbours: either one
+// launch per tile level ti+tj+tk = L (k_dilu_ro), or the whole sweep in one
+// launch, whose tiles start in level order and wait for their neighbours' faces
+// with bounded polls (k_dilu_df).  In the red-black ordering each colour is one
+// launch and nothing waits inside it.
 //   forward  y = L^-1 r :  y_e = r_e - sum_{l lower} a_el dinv_l y_l
 //   backward z = U^-1 y :  z_e = dinv_e (y_e - sum_{u upper} a_eu z_u)
 // with dinv = 1/pivot computed per frequency.  The backward sweep runs in
@@ -119,8 +121,8 @@ struct DiluArgs {
   // one coalesced read instead of 64 reads of 8 bytes, one per cache line.
   C2<T>* xf = nullptr;
   int64_t xfsys = 0, xfhalf = 0;
-  // the single-launch reference-ordered sweep (k_dilu_ro, DF): the faces in
-  // transit and the launch's counters (DfCtl)
+  // the single-launch reference-ordered sweep (k_dilu_df): the faces in transit
+  // and the launch's counters (DF_*)
   unsigned long long* mail = nullptr;
   int64_t dftiles = 0;     // tiles per active system in mail
   int* dfctl = nullptr;

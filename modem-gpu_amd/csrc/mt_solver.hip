@@ -603,8 +603,11 @@ static DiluArgs<T, V> dilu_args(const TilePlan& tp, const V* coef, int64_t cstri
 // up to nsys active systems on a tile plan; emptied here, at the start of every
 // solve (nothing is allocated where a chunk of iterations may be captured).
 constexpr int kDfSys = 16;     // active systems the mailboxes hold at most
-// items a launch takes tickets for one by one (40x40x30+10: 375 items 84 us an
-// application against 92 four by four, 750 items 97 against 95)
+// Items (tiles x systems) up to which a launch takes tickets one by one, above
+// four by four: the first spread the waves over more CUs, the second cost fewer
+// atomics.  us an application one by one / four by four: 64 tiles, 6 systems
+// 50.4 / 52.5, 8 53.9 / 53.7; 81 tiles, 6 systems 53.1 / 54.1, 8 59.5 / 55.3;
+// 375 tiles, 1 system 83 / 92, 2 96 / 94, 16 211 / 139.
 constexpr int kDfOne = 600;
 template <class T>
 static int df_prepare(mt_ctx* ctx, const TilePlan& tp, int nsys) {
@@ -630,9 +633,11 @@ static int df_check(mt_ctx* ctx) {
   return bad ? mt_fail(ctx, MT_E_DEVICE, "a DILU sweep waited in vain for a neighbouring tile") : MT_OK;
 }
 
-// One launch for the whole sweep for up to kDfSys active systems (16 at
-// 100x100x60+10: 1704 us an application against 1787; beyond, the mailboxes
-// grow and the level launches fill the chip), else one launch per tile level.
+// One launch for the whole sweep for up to kDfSys active systems, else one
+// launch per tile level, which then fills the chip (100x100x60+10, us an
+// application in one launch / by levels: 1 system 235 / 458, 8 874 / 1244, 16
+// 1698 / 1785, 20 2121 / 2094, 32 3436 / 3037.  Smaller grids would gain beyond
+// 16 too, with more mailboxes: 40x40x30+10, 24 systems 185 / 268).
 // Returns the number of launches, as every sweep function here does.
 template <class T, class V, bool FWD>
 static int dilu_ro(mt_ctx* ctx, const TilePlan& tp, DiluArgs<T, V> a) {
@@ -723,7 +728,10 @@ static int dilu_bk_apply(mt_ctx* ctx, const TilePlan& tp, DiluArgs<float, float>
   }
   int launches = 0;
   // systems per workgroup: four share a tile's couplings; fewer active ones
-  // take smaller workgroups instead of idle waves
+  // take smaller workgroups instead of idle waves (us an application with 1, 2
+  // and 4 waves, 100x100x60+10: 1 system 45.6 44.6 53.7, 2 59.6 54.0 60.4, 3 74.6
+  // 74.6 68.6, 4 99.1 86.1 81.9, 16 358 330 326; 53x61x37+9, 3 systems 27.8 28.0
+  // 26.4; at 27x23x19+7 the three are within 7 %)
   const int nw = a.nact >= 3 ? 4 : a.nact;
   for (int step = 0; step < 3; ++step) {
     const int L = (step == 1) ? 1 : 0;

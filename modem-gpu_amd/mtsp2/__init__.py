@@ -466,8 +466,9 @@ class Context:
 
     def set_dilu_variant(self, variant):
         """Launch shape of the red-black DILU sweeps: 1 one system per
-        single-wave workgroup, 4 four systems per workgroup, 5 (default) four
-        systems per workgroup in the lean LDS layout."""
+        single-wave workgroup, 4 four systems per workgroup, 5 four systems per
+        workgroup in the lean LDS layout, 6 (default) as 5 and, in the inner
+        solves on bricks, the p-update folded into the forward launches."""
         self._chk(lib().mt_set_dilu_variant(self._h, int(variant)))
 
     def set_dilu_polls(self, polls):
